@@ -11,12 +11,18 @@
 //                                     partitions of ar_model_parallel.cc:51-72
 //
 // Every stream is sequential by definition (the polar method rejects a
-// data-dependent number of draws), so the partitioned kernel runs one
-// stream per thread with the generator state in LDS, interleaved across the
-// workgroup so that every state access is bank-conflict free.  The
-// whole-grid (single stream) mode runs one workgroup that twists the state
-// in parallel chunks, evaluates 256 polar attempts at a time and compacts
-// the accepted ones with a workgroup prefix sum.
+// data-dependent number of draws), but only in two things: the recurrence of
+// its words, and the count of the pairs accepted before a place.  Which
+// kernels draw a launch's streams depends on what their records allow and on
+// how many there are (plan_noise, launch_streams):
+//   many p = 521 streams   noise_wave_kernel, four streams per wave
+//   few, long p = 521      cut into segments by jumping the generator ahead
+//                          (noise_jump_kernel), counted, then filled by
+//                          noise_wave_kernel, a row per segment
+//   few large states       words drawn ahead by one workgroup per stream
+//                          (noise_words_kernel), attempts over the whole GPU
+//   other small states     noise_seg_kernel, noise_stream_kernel
+//   many large states      noise_partitioned_kernel, one stream per thread
 //
 // All arithmetic is compiled without FP contraction, so every draw is
 // computed with the roundings the reference source writes.  The FP64 polar
@@ -25,7 +31,10 @@
 // only where the host's log is not correctly rounded.
 #include "common.hpp"
 #include "log_dd.hpp"
+#include "mt_jump.hpp"
 
+#include <algorithm>
+#include <type_traits>
 #include <vector>
 
 namespace arma_hip {
@@ -100,6 +109,28 @@ __device__ __forceinline__ float canonical_from_f(uint32_t u0) {
 	if (ret >= 1.0f) ret = 0x1.fffffep-1f;
 	return ret;
 }
+
+// One polar attempt from its words: the point and whether it is accepted.
+template <int SEM>
+struct Attempt {
+	using R = std::conditional_t<SEM == ARMA_NOISE_DOUBLE, double, float>;
+	R x, y, r2;
+	bool accept;
+	Attempt() = default;
+	__device__ __forceinline__ Attempt(const uint32_t* wv, const arma_mt_params& p) {
+		if constexpr (SEM == ARMA_NOISE_DOUBLE) {
+			const uint4 w = *reinterpret_cast<const uint4*>(wv);
+			x = 2.0 * canonical_from(mt_temper(w.x, p), mt_temper(w.y, p)) - 1.0;
+			y = 2.0 * canonical_from(mt_temper(w.z, p), mt_temper(w.w, p)) - 1.0;
+		} else {
+			const uint2 w = *reinterpret_cast<const uint2*>(wv);
+			x = 2.0f * canonical_from_f(mt_temper(w.x, p)) - 1.0f;
+			y = 2.0f * canonical_from_f(mt_temper(w.y, p)) - 1.0f;
+		}
+		r2 = x * x + y * y;
+		accept = !(r2 > R(1) || r2 == R(0));
+	}
+};
 
 template <class G>
 __device__ __forceinline__ double canonical_d(G& g) {
@@ -268,6 +299,28 @@ __global__ void mt_raw_kernel(const arma_mt_params* __restrict__ params,
 // and writes their two variates at the positions the sequential generator
 // would have given them.
 
+// Streams whose words are drawn ahead into memory (noise_words_kernel): words
+// per stream, and the blocks of kBlockAttempts attempts they hold.
+struct WordPlan {
+	int words = 0, blocks = 0;
+};
+
+// Sum of v[0 .. n-1] on every thread of the workgroup (tot: one int per wave).
+template <int THREADS>
+__device__ int block_sum(const int* v, int n, int* tot) {
+	int s = 0;
+	for (int i = threadIdx.x; i < n; i += THREADS) s += v[i];
+#pragma unroll
+	for (int m = 32; m > 0; m >>= 1) s += __shfl_xor(s, m);
+	if ((threadIdx.x & 63) == 0) tot[threadIdx.x >> 6] = s;
+	__syncthreads();
+	s = 0;
+#pragma unroll
+	for (int w = 0; w < THREADS / 64; ++w) s += tot[w];
+	__syncthreads();
+	return s;
+}
+
 template <int THREADS, int MAXNN>
 __device__ void twist_parallel(uint32_t* st, const arma_mt_params& p, int tid) {
 	constexpr int PER = (MAXNN + THREADS - 1) / THREADS;
@@ -296,7 +349,8 @@ __device__ void twist_parallel(uint32_t* st, const arma_mt_params& p, int tid) {
 
 template <class OutT, int SEM, int THREADS, int MAXNN, class Geo>
 __global__ __launch_bounds__(THREADS) void noise_stream_kernel(
-	const arma_mt_params* __restrict__ params, const uint32_t* __restrict__ seeds, Geo geo) {
+	const arma_mt_params* __restrict__ params, const uint32_t* __restrict__ seeds, Geo geo,
+	WordPlan wp, const uint32_t* __restrict__ drawn, const int* __restrict__ counts) {
 	constexpr int words_per_attempt = SEM == ARMA_NOISE_DOUBLE ? 4 : 2;
 	constexpr int round_words = THREADS * words_per_attempt;
 	constexpr int KEEP = (MAXNN + THREADS - 1) / THREADS;
@@ -346,7 +400,15 @@ __global__ __launch_bounds__(THREADS) void noise_stream_kernel(
 		}
 		out[(size_t(lo0 + t) * sy + (lo1 + x)) * sz + (lo2 + y)] = v;
 	};
-	if (tid == 0) {
+	long long produced = 0;
+	if (drawn) {
+		// what is left of a block after the words drawn for it were used up
+		// (usually nothing): the generator goes on from the last nn of them
+		produced = 2ll * block_sum<THREADS>(counts + size_t(pid) * wp.blocks, wp.blocks, wave_tot);
+		if (produced >= n) return;
+		for (int k = tid; k < p.nn; k += THREADS)
+			st[k] = drawn[size_t(pid) * wp.words + wp.words - p.nn + k];
+	} else if (tid == 0) {
 		uint32_t s = seeds ? seeds[pid] : 0u;
 		for (int k = 0; k < p.nn; ++k) {
 			st[k] = s & p.wmask;
@@ -355,7 +417,6 @@ __global__ __launch_bounds__(THREADS) void noise_stream_kernel(
 	}
 	__syncthreads();
 	int avail = 0;
-	long long produced = 0;
 	while (produced < n) {
 		while (avail < round_words) {
 			twist_parallel<THREADS, MAXNN>(st, p, tid);
@@ -419,6 +480,195 @@ __global__ __launch_bounds__(THREADS) void noise_stream_kernel(
 		}
 		avail = left;
 		__syncthreads();
+	}
+}
+
+// ---- large states: words drawn ahead, attempts over the whole GPU ----
+//
+// One workgroup that twists, tempers, transforms and stores a large-state
+// stream took 8.7 ns per normal (4.56 ms for the 524288 normals of a
+// 128x64x64 surface from one MT19937).  Only the words are sequential:
+// noise_words_kernel draws them untempered into memory, one workgroup per
+// stream, and the attempts (a fixed number of words each) are then counted
+// and transformed by workgroups of 1024 attempts, as for the segments of
+// noise_wave_kernel's streams.
+//
+// The recurrence x_(k+n) = x_(k+m) ^ y_k, y_k = y(x_k, x_(k+1)), allows n - m
+// words at a time.  Substituting it twice,
+//   x_(k+n) = x_(k+3m-2n) ^ y_(k-2(n-m)) ^ y_(k-(n-m)) ^ y_k,
+// allows min(n - 1, 3 (n - m)): 623 instead of 227 words of MT19937 per
+// workgroup barrier.
+//
+// The words drawn are those that a block needs on average; noise_stream_kernel
+// afterwards makes up what a stream's rejections left short.
+
+// y is linear over GF(2), so the three cost one: the arguments are summed
+// first.  The state moves through a straight LDS buffer (no index wraps) whose
+// tail goes back to its start when it is full.  1.34 M words of MT19937: 0.79
+// ms with three y and a ring of wrapped indices (65 VALU instructions per
+// word), 0.48 ms so, 0.22 us per chunk of 623: what remains is the chain LDS
+// read, twist, LDS write, barrier.  Several words per lane in fewer waves were
+// slower (320 lanes of two words 0.62 ms, 256 of three 0.86).
+
+constexpr int kWordThreads = 640;
+constexpr int kWordBuffer = 16384;  // words in LDS
+constexpr int kBlockAttempts = 1024, kBlockThreads = 256;
+
+__global__ __launch_bounds__(kWordThreads) void noise_words_kernel(
+	const arma_mt_params* __restrict__ params, const uint32_t* __restrict__ seeds, WordPlan wp,
+	uint32_t* __restrict__ drawn) {
+	__shared__ uint32_t buf[kWordBuffer];
+	// room for the words a chunk reads (n + 2d, d = n - m) and one chunk
+	// beyond what a move takes
+	static_assert(2 * (3 * kMaxNN) + kMaxNN <= kWordBuffer, "buffer too small");
+	const int tid = threadIdx.x;
+	const arma_mt_params p = params[blockIdx.x];
+	uint32_t* const out = drawn + size_t(blockIdx.x) * wp.words;
+	const int n = p.nn, d = p.nn - p.mm;
+	if (tid == 0) {
+		uint32_t s = seeds ? seeds[blockIdx.x] : 0u;
+		for (int k = 0; k < n; ++k) {
+			buf[k] = s & p.wmask;
+			s = 1812433253u * (s ^ (s >> 30)) + uint32_t(k + 1);
+		}
+	}
+	__syncthreads();
+	// k0 words are drawn (word j of the output is x_(n+j)) and x_(k0) is at
+	// buf[at]; single steps until 2d words lie before x_(k0)
+	int k0 = 0, at = 0;
+	const int c1 = min(d, n - 1);
+	while (k0 < wp.words && k0 < 2 * d) {
+		for (int j = tid; j < c1; j += kWordThreads) {
+			const uint32_t* x = buf + at + j;
+			const uint32_t v = mt_twist_word(x[0], x[1], x[p.mm], p);
+			buf[at + n + j] = v;
+			if (k0 + j < wp.words) out[k0 + j] = v;
+		}
+		__syncthreads();
+		k0 += c1;
+		at += c1;
+	}
+	const int c = min(n - 1, 3 * d);
+	while (k0 < wp.words) {
+		if (at + n + max(c, kWordThreads) > kWordBuffer) {
+			// x_(k0-2d) .. x_(k0+n-1) to the start of the buffer, far below
+			for (int j = tid; j < 2 * d + n; j += kWordThreads) buf[j] = buf[at - 2 * d + j];
+			__syncthreads();
+			at = 2 * d;
+		}
+		auto word = [&](int j) {
+			const uint32_t *x0 = buf + at + j, *x1 = x0 - d, *x2 = x1 - d;
+			return mt_twist_word(x0[0] ^ x1[0] ^ x2[0], x0[1] ^ x1[1] ^ x2[1], x0[n - 3 * d], p);
+		};
+		if (c <= kWordThreads && k0 + kWordThreads <= wp.words) {
+			const uint32_t v = word(tid);
+			if (tid < c) {
+				buf[at + n + tid] = v;
+				out[k0 + tid] = v;
+			}
+		} else {
+			for (int j = tid; j < c; j += kWordThreads) {
+				const uint32_t v = word(j);
+				buf[at + n + j] = v;
+				if (k0 + j < wp.words) out[k0 + j] = v;
+			}
+		}
+		__syncthreads();
+		k0 += c;
+		at += c;
+	}
+}
+
+// Pairs accepted by each block of attempts.
+template <int SEM>
+__global__ __launch_bounds__(kBlockThreads) void noise_block_count_kernel(
+	const arma_mt_params* __restrict__ params, WordPlan wp, const uint32_t* __restrict__ drawn,
+	int* __restrict__ counts) {
+	constexpr int WPA = SEM == ARMA_NOISE_DOUBLE ? 4 : 2;
+	__shared__ int tot[kBlockThreads / 64];
+	const int pid = blockIdx.y;
+	const arma_mt_params p = params[pid];
+	const uint32_t* w =
+		drawn + size_t(pid) * wp.words + size_t(blockIdx.x) * (kBlockAttempts * WPA);
+	int mine = 0;
+#pragma unroll
+	for (int a = 0; a < kBlockAttempts / kBlockThreads; ++a) {
+		const Attempt<SEM> t(w + (a * kBlockThreads + threadIdx.x) * WPA, p);
+		mine += t.accept;
+	}
+#pragma unroll
+	for (int m = 32; m > 0; m >>= 1) mine += __shfl_xor(mine, m);
+	if ((threadIdx.x & 63) == 0) tot[threadIdx.x >> 6] = mine;
+	__syncthreads();
+	if (threadIdx.x == 0) {
+		int s = 0;
+		for (int q = 0; q < kBlockThreads / 64; ++q) s += tot[q];
+		counts[size_t(pid) * wp.blocks + blockIdx.x] = s;
+	}
+}
+
+// The normals of each block of attempts, from the position that the counts of
+// the stream's earlier blocks give it.
+template <class OutT, int SEM, class Geo>
+__global__ __launch_bounds__(kBlockThreads) void noise_block_fill_kernel(
+	const arma_mt_params* __restrict__ params, Geo geo, WordPlan wp,
+	const uint32_t* __restrict__ drawn, const int* __restrict__ counts) {
+	constexpr int WPA = SEM == ARMA_NOISE_DOUBLE ? 4 : 2;
+	constexpr int A = kBlockAttempts / kBlockThreads;
+	__shared__ int tot[A][kBlockThreads / 64];
+	__shared__ double ltab[kLogDdRows * 3];
+	stage_log_table(ltab);
+	const int pid = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	const StreamBlock<OutT> blk = geo(pid);
+	const long long e12 = (long long)blk.e1 * blk.e2, n = blk.e0 * e12;
+	const long long before = 2ll * block_sum<kBlockThreads>(counts + size_t(pid) * wp.blocks,
+	                                                        int(blockIdx.x), tot[0]);
+	if (before >= n) return;
+	const arma_mt_params p = params[pid];
+	const uint32_t* w =
+		drawn + size_t(pid) * wp.words + size_t(blockIdx.x) * (kBlockAttempts * WPA);
+	Attempt<SEM> t[A];
+	int below[A];
+#pragma unroll
+	for (int a = 0; a < A; ++a) {
+		t[a] = Attempt<SEM>(w + (a * kBlockThreads + threadIdx.x) * WPA, p);
+		const unsigned long long mask = __ballot(t[a].accept);
+		below[a] = __popcll(mask & ((1ull << lane) - 1ull));
+		if (lane == 0) tot[a][wave] = __popcll(mask);
+	}
+	__syncthreads();
+	int run = 0;
+#pragma unroll
+	for (int a = 0; a < A; ++a)
+		for (int q = 0; q < kBlockThreads / 64; ++q) {
+			if (q == wave) below[a] += run;
+			run += tot[a][q];
+		}
+	auto put = [&](long long q, OutT v) {
+		const uint32_t t0 = uint32_t(q) / uint32_t(e12), r = uint32_t(q) - t0 * uint32_t(e12);
+		const uint32_t x = r / uint32_t(blk.e2);
+		blk.out[(size_t(blk.lo0 + t0) * blk.sy + (blk.lo1 + x)) * blk.sz +
+		        (blk.lo2 + (r - x * uint32_t(blk.e2)))] = v;
+	};
+#pragma unroll
+	for (int a = 0; a < A; ++a) {
+		const long long pos = before + 2ll * below[a];
+		double v0, v1;
+		if (SEM == ARMA_NOISE_DOUBLE) {
+			const double r2 = t[a].accept ? double(t[a].r2) : 0.5;
+			const double mult = sqrt(-2.0 * log_dd(r2, ltab) / r2);
+			v0 = t[a].y * mult * blk.sd + 0.0;
+			v1 = t[a].x * mult * blk.sd + 0.0;
+		} else {
+			const float r2 = t[a].accept ? float(t[a].r2) : 0.5f;
+			const float mult = sqrtf(-2.0f * logf(r2) / r2);
+			v0 = float(t[a].y) * mult * blk.sdf + 0.0f;
+			v1 = float(t[a].x) * mult * blk.sdf + 0.0f;
+		}
+		if (t[a].accept && pos < n) {
+			put(pos, OutT(v0));
+			if (pos + 1 < n) put(pos + 1, OutT(v1));
+		}
 	}
 }
 
@@ -632,10 +882,53 @@ __device__ __forceinline__ uint32_t mt_twist_y(uint32_t a, uint32_t b, const arm
 	return (x >> 1) ^ ((x & 1u) ? p.aaa : 0u);
 }
 
-template <class OutT, int SEM, class Geo>
+// The state of one stream on a 16-lane row and its twist.
+struct Twist521 {
+	uint32_t s, t;
+	__device__ __forceinline__ void next(int k, const arma_mt_params& p) {
+		const uint32_t nx1 = row_move_or<kRowShl1>(t, s);  // old[k + 1]; lane 15: old[16]
+		const uint32_t t8 = row_move<kRowShl7>(t);          // lane 8 <- old[16]
+		const uint32_t nx8 = row_move_or<kRowShl8>(t8, s);  // old[k + 8]; lane 8: old[16]
+		const uint32_t y = mt_twist_y(s, nx1, p);
+		const uint32_t a = nx8 ^ y;                  // new[k], k <= 8
+		const uint32_t a9 = row_move<kRowShr9>(a);   // new[k - 9]
+		const uint32_t a0 = row_move<kRowShr15>(a);  // lane 15 <- new[0]
+		const uint32_t a7 = row_move<kRowShr8>(a);   // lane 15 <- new[7]
+		t = a7 ^ mt_twist_y(t, a0, p);               // new[16] (lane 15)
+		s = k <= kWaveMM ? a : (a9 ^ y);
+	}
+};
+
+// Orders a wave's LDS stores before its later loads of them (LDS operations
+// of one wave complete in order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_order() {
+	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// How streams are cut: per_stream segments at most, of L = e0 2^squarings
+// words (rounds rounds of kRoundWords) each, the last one open-ended.
+struct SegmentPlan {
+	int per_stream = 1, e0 = 0, squarings = 0, rounds = 0;
+	// Segments of a stream of n normals: its expected words (a pair takes
+	// 4 / pi attempts on average) over the segment length, rounded up.
+	__host__ __device__ int segments(long long n, int words_per_attempt) const {
+		const long long words = (n * words_per_attempt * 41722 >> 16) + 1;
+		const long long len = (long long)rounds * kRoundWords;
+		const long long k = (words + len - 1) / len;
+		return k < 1 ? 1 : k < per_stream ? int(k) : per_stream;
+	}
+};
+
+// SEG: a row's work is not a whole stream but one of the segments a long
+// stream is cut into (see noise_jump_kernel).  Every segment but a stream's
+// last is seg.rounds rounds long; the last runs until the block is full.
+template <class OutT, int SEM, bool SEG, class Geo>
 __global__ __launch_bounds__(kPcThreads) void noise_wave_kernel(
 	const arma_mt_params* __restrict__ params, const uint32_t* __restrict__ seeds, Geo geo,
-	int nstreams) {
+	int nstreams, SegmentPlan seg, const uint32_t* __restrict__ states,
+	const int* __restrict__ counts) {
 	constexpr int WPA = SEM == ARMA_NOISE_DOUBLE ? 4 : 2;  // words per attempt
 	constexpr int A = kRoundWords / (16 * WPA);            // attempts per lane per round
 	static_assert(A * 16 * WPA == kRoundWords, "a round is whole attempts");
@@ -650,25 +943,19 @@ __global__ __launch_bounds__(kPcThreads) void noise_wave_kernel(
 	const int row = lane >> 4, k = lane & 15;
 	const int g = wave & 3;
 	const bool producer = ((wave >> 2) ^ (wave & 1)) == 0;
-	const int pid = (int(blockIdx.x) * 4 + g) * 4 + row;
+	const int rid = (int(blockIdx.x) * 4 + g) * 4 + row;
+	const int pid = !SEG ? rid : rid / seg.per_stream;
+	const int sid = !SEG ? 0 : rid - pid * seg.per_stream;
 	const bool valid = pid < nstreams;
 	uint32_t* ring = ring_all[g][row];
 	const arma_mt_params p = params[valid ? pid : 0];
 
 	// producer: the state (lane k: word k; word 16 on lane 15, held by all)
-	uint32_t s = 0, t = 0;
+	Twist521 tw{0, 0};
+	uint32_t &s = tw.s, &t = tw.t;
 	int wpos = 0;
 	auto twist = [&]() {
-		const uint32_t nx1 = row_move_or<kRowShl1>(t, s);  // old[k + 1]; lane 15: old[16]
-		const uint32_t t8 = row_move<kRowShl7>(t);          // lane 8 <- old[16]
-		const uint32_t nx8 = row_move_or<kRowShl8>(t8, s);  // old[k + 8]; lane 8: old[16]
-		const uint32_t y = mt_twist_y(s, nx1, p);
-		const uint32_t a = nx8 ^ y;                  // new[k], k <= 8
-		const uint32_t a9 = row_move<kRowShr9>(a);   // new[k - 9]
-		const uint32_t a0 = row_move<kRowShr15>(a);  // lane 15 <- new[0]
-		const uint32_t a7 = row_move<kRowShr8>(a);   // lane 15 <- new[7]
-		t = a7 ^ mt_twist_y(t, a0, p);               // new[16] (lane 15)
-		s = k <= kWaveMM ? a : (a9 ^ y);
+		tw.next(k, p);
 		ring[(wpos + k) & (kRingWords - 1)] = s;
 		if (k == 15) ring[(wpos + 16) & (kRingWords - 1)] = t;
 		wpos += kWaveNN;
@@ -683,7 +970,15 @@ __global__ __launch_bounds__(kPcThreads) void noise_wave_kernel(
 	const double stddev = blk.sd;
 	const float stddev_f = blk.sdf;
 	const long long e12 = (long long)blk.e1 * e2;
-	const long long n = valid ? (long long)blk.e0 * e12 : 0;
+	long long n = valid ? (long long)blk.e0 * e12 : 0;
+	// rounds of this row: unbounded (until the block is full) for a whole
+	// stream and a stream's last segment
+	int rounds = 0x7fffffff;
+	if constexpr (SEG) {
+		const int nseg = seg.segments(n, WPA);
+		if (sid < nseg - 1) rounds = seg.rounds;
+		if (sid > nseg - 1) n = 0;
+	}
 	const double r12 = 1.0 / double(e12), r2 = 1.0 / double(e2);
 	const bool pow2 = (e2 & (e2 - 1)) == 0 && (e12 & (e12 - 1)) == 0;
 	const int s2 = __ffs(unsigned(e2)) - 1, s12 = __ffsll((unsigned long long)e12) - 1;
@@ -715,6 +1010,16 @@ __global__ __launch_bounds__(kPcThreads) void noise_wave_kernel(
 		if (q + 1 < n) out[even_rows ? i0 + 1 : index(q + 1)] = v1;
 	};
 	long long produced = 0;
+	if constexpr (SEG) {
+		// the pairs of the stream's earlier segments
+		if (!producer && n > 0) {
+			int before = 0;
+			for (int i = k; i < sid; i += 16) before += counts[rid - sid + i];
+#pragma unroll
+			for (int m = 8; m > 0; m >>= 1) before += __shfl_xor(before, m, 16);
+			produced = 2ll * before;
+		}
+	}
 	auto consume = [&](int r) {
 		// attempts a * 16 + k (a < A) of the row's stream in round r; the
 		// transform is evaluated on every lane (a rejected attempt on a
@@ -744,6 +1049,7 @@ __global__ __launch_bounds__(kPcThreads) void noise_wave_kernel(
 		int total = 0;
 #pragma unroll
 		for (int a = 0; a < A; ++a) {
+			if constexpr (SEG) acc[a] = acc[a] && r < rounds;
 			const uint32_t bits = uint32_t(__ballot(acc[a]) >> (16 * row)) & 0xffffu;
 			below[a] = total + __popc(bits & ((1u << k) - 1u));
 			total += __popc(bits);
@@ -770,12 +1076,17 @@ __global__ __launch_bounds__(kPcThreads) void noise_wave_kernel(
 	if (producer) {
 		// sgenrand_mt: word w of the recurrence from the seed; lane k keeps
 		// word k, every lane keeps word 16 (lane 15's copy is the one used)
-		uint32_t x = valid && seeds ? seeds[pid] : 0u;
-		for (int w = 0; w < kWaveNN; ++w) {
-			const uint32_t v = x & p.wmask;
-			if (w == k) s = v;
-			if (w == kWaveNN - 1) t = v;
-			x = 1812433253u * (x ^ (x >> 30)) + uint32_t(w + 1);
+		if constexpr (!SEG) {
+			uint32_t x = valid && seeds ? seeds[pid] : 0u;
+			for (int w = 0; w < kWaveNN; ++w) {
+				const uint32_t v = x & p.wmask;
+				if (w == k) s = v;
+				if (w == kWaveNN - 1) t = v;
+				x = 1812433253u * (x ^ (x >> 30)) + uint32_t(w + 1);
+			}
+		} else if (n > 0) {
+			s = states[size_t(rid) * kWaveNN + k];
+			t = states[size_t(rid) * kWaveNN + kWaveNN - 1];
 		}
 		while (wpos < kRoundWords) twist();
 	}
@@ -785,7 +1096,9 @@ __global__ __launch_bounds__(kPcThreads) void noise_wave_kernel(
 			while (wpos < (r + 2) * kRoundWords) twist();  // round r + 1
 		} else {
 			consume(r);
-			const bool mine_done = !__any(produced < n);
+			bool more = produced < n;
+			if constexpr (SEG) more = more && r + 1 < rounds;
+			const bool mine_done = !__any(more);
 			if (lane == 0) gdone[r & 1][g] = mine_done;
 		}
 		__syncthreads();
@@ -793,10 +1106,354 @@ __global__ __launch_bounds__(kPcThreads) void noise_wave_kernel(
 	}
 }
 
+// ---- long MT521 streams cut into segments ----
+//
+// With few streams the launch time of noise_wave_kernel is the length of one
+// stream (29 ns per normal: a twist is a dependent chain), whatever the GPU
+// could do beside it: 2.12 ms for streams of 73728 normals, one or 4096 of
+// them.  Cut in segments, 64 such streams take 0.18 ms, 1000 0.79 ms.  A polar attempt always takes the same number of words,
+// accepted or not, so a stream's words can be cut anywhere between attempts
+// once the generator's state there is known: segment j of a stream starts
+// at its word j L.
+//
+// noise_jump_kernel finds those states, one workgroup per stream.  With the
+// residue g = t^(mL) mod chi (mt_jump.hpp) the state m segments further on is
+// a correlation of g with the 538 words after a segment's start, so the
+// states double in number per level: from segments 0..m-1 to m..2m-1, g
+// squared in between.  Each 16-lane row twists one segment's 538 words into
+// LDS and correlates them (lane k: state word k, lane 15 also word 16).
+// noise_count_kernel then counts what each segment accepts, and
+// noise_wave_kernel writes the normals of all segments side by side, each
+// from the sum of the counts before it.  The words, and so the noise, are
+// those of the sequential generator.
+
+// Streams cut into at most this many segments take one-wave workgroups, many
+// per CU: their polynomial work is what costs, not the segments.
+constexpr int kJumpFew = 8;
+// words of a row's window: 521 + 17 rounded up to whole twists; the row
+// stride keeps a wave's four rows on different banks
+constexpr int kJumpWindow = 544, kJumpStride = 560;
+
+__constant__ const JumpTable kJumpPolys = jump_table();
+
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void noise_jump_kernel(
+	const arma_mt_params* __restrict__ params, const uint32_t* __restrict__ seeds,
+	SegmentPlan seg, uint32_t* __restrict__ states) {
+	constexpr int kRows = THREADS / 16;
+	constexpr int kGroups = THREADS / kJumpWords < 8 ? THREADS / kJumpWords : 8;
+	__shared__ uint32_t win[kRows][kJumpStride];
+	__shared__ uint32_t shift[32][kJumpWords];  // t^(521 + b) mod chi
+	__shared__ uint32_t sq[2 * kJumpWords + 2];
+	__shared__ uint32_t g[kJumpWords];
+	const int tid = threadIdx.x;
+	const int row = tid >> 4, k = tid & 15;
+	const arma_mt_params p = params[blockIdx.x];
+	uint32_t* const st = states + size_t(blockIdx.x) * seg.per_stream * kWaveNN;
+	if (tid == 0) {
+		// sgenrand_mt: the state of segment 0
+		uint32_t x = seeds ? seeds[blockIdx.x] : 0u;
+		for (int w = 0; w < kWaveNN; ++w) {
+			st[w] = x & p.wmask;
+			x = 1812433253u * (x ^ (x >> 30)) + uint32_t(w + 1);
+		}
+	}
+	if (seg.per_stream == 1) return;
+	// t^521 mod chi
+	if (tid < kJumpWords) {
+		uint32_t v = kJumpPolys.base.w[tid];
+		for (int i = 0; i < 32; ++i) v ^= ((p.aaa >> i) & 1u) ? kJumpPolys.a[i].w[tid] : 0u;
+		shift[0][tid] = v;
+		// t^e0, e0 at most 512
+		g[tid] = seg.e0 >> 5 == tid ? 1u << (seg.e0 & 31) : 0u;
+	}
+	__syncthreads();
+	for (int b = 1; b < 32; ++b) {
+		if (tid < kJumpWords) {
+			const uint32_t top = (shift[b - 1][kJumpWords - 1] >> (kJumpTop - 1)) & 1u;
+			uint32_t v = (shift[b - 1][tid] << 1) | (tid ? shift[b - 1][tid - 1] >> 31 : 0u);
+			if (tid == kJumpWords - 1) v &= (1u << kJumpTop) - 1u;
+			shift[b][tid] = v ^ (top ? shift[0][tid] : 0u);
+		}
+		__syncthreads();
+	}
+	// g <- g^2 mod chi
+	auto square = [&]() {
+		if (tid < kJumpWords) {
+			// bit i to bit 2 i
+			auto spread = [](uint32_t v) {
+				v = (v | (v << 8)) & 0x00ff00ffu;
+				v = (v | (v << 4)) & 0x0f0f0f0fu;
+				v = (v | (v << 2)) & 0x33333333u;
+				return (v | (v << 1)) & 0x55555555u;
+			};
+			sq[2 * tid] = spread(g[tid] & 0xffffu);
+			sq[2 * tid + 1] = spread(g[tid] >> 16);
+		}
+		__syncthreads();
+		// 32 bits at a time from the top (the square has degree at most 1040):
+		// bits 521 + 32c .. 521 + 32c + 31 select rows of shift
+		for (int c = 16; c >= 0; --c) {
+			const uint32_t v =
+				(sq[16 + c] >> kJumpTop) | (sq[17 + c] << (32 - kJumpTop));
+			__syncthreads();
+			if (tid < kGroups * kJumpWords) {
+				const int w = tid % kJumpWords, b0 = tid / kJumpWords;
+				uint32_t x = 0;
+#pragma unroll
+				for (int q = 0; q < (32 + kGroups - 1) / kGroups; ++q) {
+					const int b = min(b0 + kGroups * q, 31);
+					x ^= b0 + kGroups * q < 32 && ((v >> b) & 1u) ? shift[b][w] : 0u;
+				}
+				if (x) atomicXor(&sq[c + w], x);
+			}
+			__syncthreads();
+		}
+		if (tid < kJumpWords)
+			g[tid] = tid == kJumpWords - 1 ? sq[tid] & ((1u << kJumpTop) - 1u) : sq[tid];
+		__syncthreads();
+	};
+	for (int q = 0; q < seg.squarings; ++q) square();
+	uint32_t* const mine = win[row];
+	for (int m = 1; m < seg.per_stream; m *= 2) {
+		if (m > 1) square();
+		for (int t0 = m; t0 < min(2 * m, seg.per_stream); t0 += kRows) {
+			const int to = t0 + row;
+			const bool act = to < min(2 * m, seg.per_stream);
+			if (!__any(act)) continue;
+			const uint32_t* const from = st + size_t(act ? to - m : 0) * kWaveNN;
+			Twist521 tw{from[k], from[kWaveNN - 1]};
+			mine[k] = tw.s;
+			if (k == 15) mine[16] = tw.t;
+			for (int w = kWaveNN; w < kJumpWindow; w += kWaveNN) {
+				tw.next(k, p);
+				mine[w + k] = tw.s;
+				if (k == 15) mine[w + 16] = tw.t;
+			}
+			wave_lds_order();
+			// state word k: sum of g_i x_(i+k); word 16 one word behind on lane 15
+			uint32_t acc = 0, acc16 = 0, prev = 0;
+			for (int w = 0; w < kJumpWords; ++w) {
+				const uint32_t gw = __builtin_amdgcn_readfirstlane(g[w]);
+				const uint32_t* x = mine + 32 * w + k;
+				if (w < kJumpWords - 1) {
+#pragma unroll
+					for (int b = 0; b < 32; ++b) {
+						const uint32_t mask = 0u - ((gw >> b) & 1u);
+						acc ^= x[b] & mask;
+						acc16 ^= x[b] & prev;
+						prev = mask;
+					}
+				} else {
+#pragma unroll
+					for (int b = 0; b < kJumpTop; ++b) {
+						const uint32_t mask = 0u - ((gw >> b) & 1u);
+						acc ^= x[b] & mask;
+						acc16 ^= x[b] & prev;
+						prev = mask;
+					}
+					acc16 ^= x[kJumpTop] & prev;
+				}
+			}
+			if (act) {
+				st[size_t(to) * kWaveNN + k] = acc;
+				if (k == 15) st[size_t(to) * kWaveNN + 16] = acc16;
+			}
+			wave_lds_order();
+		}
+		__syncthreads();  // the level's states are the next level's starts
+	}
+}
+
+// Pairs that each segment but a stream's last accepts.  Four segments per
+// wave, one per 16-lane row; a wave twists a round of words of its rows into
+// LDS and tests their attempts, without the producer and consumer roles of
+// noise_wave_kernel: the twists are most of the work and the waves of a
+// SIMD fill each other's stalls.  In FP64 semantics an attempt is decided by
+// the high words of its two uniforms (each within 2^-31 of the uniform's
+// value, so r^2 within 2^-28) unless r^2 is that close to 1 or may be zero.
+constexpr int kCountRows = 16;  // rows per workgroup
+
+template <int SEM, class Geo>
+__global__ __launch_bounds__(16 * kCountRows) void noise_count_kernel(
+	const arma_mt_params* __restrict__ params, Geo geo, int nstreams, SegmentPlan seg,
+	const uint32_t* __restrict__ states, int* __restrict__ counts) {
+	constexpr int WPA = SEM == ARMA_NOISE_DOUBLE ? 4 : 2;
+	constexpr int A = kRoundWords / (16 * WPA);
+	constexpr int kRing = 512;  // a round and the 16 words written ahead
+	__shared__ __align__(16) uint32_t ring_all[kCountRows][kRing + 16];
+	const int lrow = threadIdx.x >> 4, k = threadIdx.x & 15;
+	const int rid = int(blockIdx.x) * kCountRows + lrow;
+	const int pid = rid / seg.per_stream, sid = rid - pid * seg.per_stream;
+	bool live = false;
+	if (pid < nstreams) {
+		const auto blk = geo(pid);
+		live = sid < seg.segments((long long)blk.e0 * blk.e1 * blk.e2, WPA) - 1;
+	}
+	if (!__any(live)) return;
+	const arma_mt_params p = params[live ? pid : 0];
+	uint32_t* const ring = ring_all[lrow];
+	Twist521 tw{0, 0};
+	if (live) {
+		tw.s = states[size_t(rid) * kWaveNN + k];
+		tw.t = states[size_t(rid) * kWaveNN + kWaveNN - 1];
+	}
+	const int row = lrow & 3;  // of the wave
+	int wpos = 0, total = 0;
+	for (int r = 0; r < seg.rounds; ++r) {
+		while (wpos < (r + 1) * kRoundWords) {
+			tw.next(k, p);
+			ring[(wpos + k) & (kRing - 1)] = tw.s;
+			if (k == 15) ring[(wpos + 16) & (kRing - 1)] = tw.t;
+			wpos += kWaveNN;
+		}
+		wave_lds_order();
+		const uint32_t* words = ring + ((r * kRoundWords) & (kRing - 1));
+		bool acc[A];
+#pragma unroll
+		for (int a = 0; a < A; ++a) {
+			const uint32_t* wv = words + (a * 16 + k) * WPA;
+			if (SEM == ARMA_NOISE_DOUBLE) {
+				const uint4 w = *reinterpret_cast<const uint4*>(wv);
+				const uint32_t u = mt_temper(w.y, p), v = mt_temper(w.w, p);
+				const double x = double(int(u ^ 0x80000000u)), y = double(int(v ^ 0x80000000u));
+				const double q = fma(x, x, y * y);  // r^2 * 2^62
+				acc[a] = q <= 0x1p62;
+				if (__builtin_expect(fabs(q - 0x1p62) < 0x1p35 || q < 0x1p12, 0)) {
+					const double xd = 2.0 * canonical_from(mt_temper(w.x, p), u) - 1.0;
+					const double yd = 2.0 * canonical_from(mt_temper(w.z, p), v) - 1.0;
+					const double r2 = xd * xd + yd * yd;
+					acc[a] = !(r2 > 1.0 || r2 == 0.0);
+				}
+			} else {
+				const uint2 w = *reinterpret_cast<const uint2*>(wv);
+				const float x = 2.0f * canonical_from_f(mt_temper(w.x, p)) - 1.0f;
+				const float y = 2.0f * canonical_from_f(mt_temper(w.y, p)) - 1.0f;
+				const float r2 = x * x + y * y;
+				acc[a] = !(r2 > 1.0f || r2 == 0.0f);
+			}
+		}
+#pragma unroll
+		for (int a = 0; a < A; ++a)
+			total += __popc(uint32_t(__ballot(acc[a]) >> (16 * row)) & 0xffffu);
+		wave_lds_order();
+	}
+	if (live && k == 0) counts[rid] = total;
+}
+
 bool wave_kernel_fits(const arma_mt_params* mts, int n) {
 	for (int i = 0; i < n; ++i)
 		if (mts[i].nn != kWaveNN || mts[i].mm != kWaveMM) return false;
 	return true;
+}
+
+// Streams whose states noise_jump_kernel can advance: the records of p = 521
+// with the dynamic creator's masks.
+bool jump_fits(const arma_mt_params* mts, int n) {
+	for (int i = 0; i < n; ++i) {
+		const arma_mt_params& q = mts[i];
+		if (q.nn != kJumpN || q.mm != kJumpM || q.umask != 0xffffffffu << kJumpR ||
+		    q.lmask != ~(0xffffffffu << kJumpR))
+			return false;
+	}
+	return true;
+}
+
+// Rows a segmented launch aims at (two workgroups of 16 rows per CU), the
+// most segments of one stream, and the shortest segment in words.
+// Rows a segmented launch aims at (two workgroups of 16 rows per CU), the
+// most segments of one stream, and the shortest segment in words.
+constexpr int kSegRowsPerCu = 32, kMaxSegments = 256, kMinSegmentWords = 1024;
+// Measured on MI355X, in ns: per word of a row filling its block and counting
+// (one workgroup of rows per CU), the jump's fixed part, each of its levels
+// or squarings, and its share per stream where many jump side by side.
+constexpr double kWordNs = 11.4, kCountWordNs = 4.5, kJumpNs = 30e3, kJumpLevelNs = 6e3,
+                 kJumpStreamNs = 40.0;
+
+// How to cut nstreams streams whose longest block has n normals.
+SegmentPlan plan_segments(const arma_hip_ctx* ctx, int sem, int nstreams, long long n,
+                          const arma_mt_params* mts, bool small_blocks) {
+	SegmentPlan seg;
+	const int wpa = sem == ARMA_NOISE_DOUBLE ? 4 : 2;
+	const int rows = kSegRowsPerCu * std::max(ctx->num_cus, 1);
+	const int most = std::min(kMaxSegments, rows / std::max(nstreams, 1));
+	if (!small_blocks || most < 2 || !jump_fits(mts, nstreams)) return seg;
+	// segment lengths e0 2^q, whole rounds of words: the shortest that keeps
+	// the launch within rows
+	for (int q = 2; q < 40; ++q)
+		for (int e0 : {256, 320, 384, 448}) {
+			const long long len = (long long)e0 << q;
+			if (len < kMinSegmentWords || len > (1ll << 30)) continue;
+			seg.e0 = e0;
+			seg.squarings = q;
+			seg.rounds = int(len / kRoundWords);
+			seg.per_stream = kMaxSegments + 1;
+			const int k = seg.segments(n, wpa);
+			if (k > most) continue;
+			seg.per_stream = k;
+			int levels = 0;
+			while ((1 << levels) < k) ++levels;
+			const double words = double(n) * wpa * 0.6366;
+			const double whole = kWordNs * words;
+			// two workgroups on a CU share its issue slots
+			const double share =
+				std::max(1.0, 0.85 * 2.0 * double(nstreams) * k / double(rows));
+			const double cut = kJumpNs + kJumpLevelNs * (levels + q) + kJumpStreamNs * nstreams +
+			                   (kWordNs + kCountWordNs) * double(len) * share;
+			// one stream of 32768 normals: 146 us cut in 82 against 905 whole;
+			// 1000 of 73728: 0.79 against 2.12 ms; 2700 of 8192, which this
+			// line leaves whole, 279 against 241 us
+			if (k < 2 || cut > 0.93 * whole) return SegmentPlan();
+			return seg;
+		}
+	return SegmentPlan();
+}
+
+// Streams of large states take their words from noise_words_kernel when they
+// have at least kAheadNormals normals (below, the extra launches cost what the
+// stream does) and all words fit kAheadBytes.
+constexpr long long kAheadNormals = 8192, kAheadBytes = 256ll << 20;
+
+WordPlan plan_ahead(const arma_hip_ctx* ctx, int sem, int nstreams, long long n,
+                    const arma_mt_params* mts, bool small_blocks) {
+	WordPlan wp;
+	int nn_max = 0;
+	for (int i = 0; i < nstreams; ++i) nn_max = std::max(nn_max, int(mts[i].nn));
+	if (!small_blocks || nn_max <= 64 || n < kAheadNormals ||
+	    nstreams > 4 * std::max(ctx->num_cus, 1))
+		return wp;
+	const int wpa = sem == ARMA_NOISE_DOUBLE ? 4 : 2;
+	// 4 / pi attempts per pair on average, in whole blocks
+	const long long blocks = (n * 41722 / 65536 + kBlockAttempts) / kBlockAttempts;
+	const long long words = blocks * kBlockAttempts * wpa;
+	if (words * 4 * nstreams > kAheadBytes || blocks > 65535) return wp;
+	wp.words = int(words);
+	wp.blocks = int(blocks);
+	return wp;
+}
+
+// How a launch draws its streams: whole (neither set), by segments, or with
+// the words drawn ahead.
+struct NoisePlan {
+	SegmentPlan seg;
+	WordPlan ahead;
+	// device bytes beside the parameters and seeds
+	size_t bytes(int nstreams) const {
+		if (ahead.words > 0)
+			return size_t(nstreams) * (size_t(ahead.words) + ahead.blocks) * sizeof(uint32_t);
+		if (seg.per_stream > 1)
+			return size_t(nstreams) * seg.per_stream * (kWaveNN + 1) * sizeof(uint32_t);
+		return 0;
+	}
+};
+
+NoisePlan plan_noise(const arma_hip_ctx* ctx, int sem, int nstreams, long long n,
+                     const arma_mt_params* mts, bool small_blocks) {
+	NoisePlan plan;
+	plan.ahead = plan_ahead(ctx, sem, nstreams, n, mts, small_blocks);
+	if (plan.ahead.words == 0)
+		plan.seg = plan_segments(ctx, sem, nstreams, n, mts, small_blocks);
+	return plan;
 }
 
 // The two-per-wave kernel applies to states of at most 32 words whose twist
@@ -824,34 +1481,72 @@ void validate_params(const arma_mt_params* mts, int n) {
 	}
 }
 
-// Launches the noise of nstreams streams whose output blocks geo describes,
-// with the kernel their parameter sets allow: a whole workgroup for a single
-// stream, two streams per wave for small dcmt states, one wave per stream up
-// to 64 state words, one workgroup per stream for a few large states, else
-// one thread per stream.
+// Launches the noise of nstreams streams whose output blocks geo describes:
+// as the plan says, or whole streams with the kernel their parameter sets
+// allow: four streams per wave for p = 521, a whole workgroup for another
+// single stream, two streams per wave for small dcmt states, one wave per
+// stream up to 64 state words, one workgroup per stream for a few large
+// states, else one thread per stream.
 template <class OutT, int SEM, class Geo>
 void launch_streams(arma_hip_ctx* ctx, const arma_mt_params* hparams,
                     const arma_mt_params* dparams, const uint32_t* dseeds, Geo geo, int nstreams,
-                    bool small_blocks) {
+                    bool small_blocks, const NoisePlan& plan, void* buf) {
+	const SegmentPlan& seg = plan.seg;
+	const WordPlan& wp = plan.ahead;
+	if (wp.words > 0) {
+		uint32_t* drawn = (uint32_t*)buf;
+		int* counts = (int*)(drawn + size_t(nstreams) * wp.words);
+		noise_words_kernel<<<nstreams, kWordThreads, 0, ctx->stream>>>(dparams, dseeds, wp, drawn);
+		ARMA_HIP_CHECK(hipGetLastError());
+		noise_block_count_kernel<SEM><<<dim3(wp.blocks, nstreams), kBlockThreads, 0, ctx->stream>>>(
+			dparams, wp, drawn, counts);
+		ARMA_HIP_CHECK(hipGetLastError());
+		noise_block_fill_kernel<OutT, SEM, Geo>
+			<<<dim3(wp.blocks, nstreams), kBlockThreads, 0, ctx->stream>>>(dparams, geo, wp, drawn,
+			                                                           counts);
+		ARMA_HIP_CHECK(hipGetLastError());
+		noise_stream_kernel<OutT, SEM, 256, kMaxNN, Geo>
+			<<<nstreams, 256, 0, ctx->stream>>>(dparams, dseeds, geo, wp, drawn, counts);
+		ARMA_HIP_CHECK(hipGetLastError());
+		return;
+	}
+	if (seg.per_stream > 1) {
+		const int rows = nstreams * seg.per_stream;
+		uint32_t* states = (uint32_t*)buf;
+		int* counts = (int*)(states + size_t(rows) * kWaveNN);
+		if (seg.per_stream <= kJumpFew)
+			noise_jump_kernel<64><<<nstreams, 64, 0, ctx->stream>>>(dparams, dseeds, seg, states);
+		else
+			noise_jump_kernel<512><<<nstreams, 512, 0, ctx->stream>>>(dparams, dseeds, seg, states);
+		ARMA_HIP_CHECK(hipGetLastError());
+		noise_count_kernel<SEM, Geo><<<div_ceil(rows, kCountRows), 16 * kCountRows, 0, ctx->stream>>>(
+			dparams, geo, nstreams, seg, states, counts);
+		ARMA_HIP_CHECK(hipGetLastError());
+		noise_wave_kernel<OutT, SEM, true, Geo>
+			<<<div_ceil(rows, 16), kPcThreads, 0, ctx->stream>>>(dparams, dseeds, geo, nstreams,
+			                                                   seg, states, counts);
+		ARMA_HIP_CHECK(hipGetLastError());
+		return;
+	}
 	int nn_max = 0;
 	for (int i = 0; i < nstreams; ++i) nn_max = std::max(nn_max, int(hparams[i].nn));
-	if (nstreams == 1) {
+	if (small_blocks && wave_kernel_fits(hparams, nstreams)) {
+		noise_wave_kernel<OutT, SEM, false, Geo>
+			<<<div_ceil(nstreams, 16), kPcThreads, 0, ctx->stream>>>(dparams, dseeds, geo,
+			                                                       nstreams, seg, nullptr, nullptr);
+	} else if (nstreams == 1) {
 		// the whole grid from one stream (framework=none)
 		noise_stream_kernel<OutT, SEM, 256, kMaxNN, Geo>
-			<<<1, 256, 0, ctx->stream>>>(dparams, dseeds, geo);
-	} else if (small_blocks && wave_kernel_fits(hparams, nstreams)) {
-		noise_wave_kernel<OutT, SEM, Geo>
-			<<<div_ceil(nstreams, 16), kPcThreads, 0, ctx->stream>>>(dparams, dseeds, geo,
-			                                                       nstreams);
+			<<<1, 256, 0, ctx->stream>>>(dparams, dseeds, geo, wp, nullptr, nullptr);
 	} else if (small_blocks && seg_kernel_fits(hparams, nstreams)) {
 		noise_seg_kernel<OutT, SEM, Geo>
 			<<<div_ceil(nstreams, 2), 64, 0, ctx->stream>>>(dparams, dseeds, geo, nstreams);
 	} else if (nn_max <= 64) {
 		noise_stream_kernel<OutT, SEM, 64, 64, Geo>
-			<<<nstreams, 64, 0, ctx->stream>>>(dparams, dseeds, geo);
+			<<<nstreams, 64, 0, ctx->stream>>>(dparams, dseeds, geo, wp, nullptr, nullptr);
 	} else if (nstreams <= 4 * std::max(ctx->num_cus, 1)) {
 		noise_stream_kernel<OutT, SEM, 256, kMaxNN, Geo>
-			<<<nstreams, 256, 0, ctx->stream>>>(dparams, dseeds, geo);
+			<<<nstreams, 256, 0, ctx->stream>>>(dparams, dseeds, geo, wp, nullptr, nullptr);
 	} else {
 		const int tpb = std::min(threads_for_state(nn_max), 64);
 		noise_partitioned_kernel<OutT, SEM, Geo>
@@ -864,23 +1559,24 @@ void launch_streams(arma_hip_ctx* ctx, const arma_mt_params* hparams,
 template <class Geo2>
 void launch_by_type(arma_hip_ctx* ctx, bool fp32, int sem, const arma_mt_params* hparams,
                     const arma_mt_params* dparams, const uint32_t* dseeds, void* out,
-                    const Geo2& g, int nstreams, bool small_blocks) {
+                    const Geo2& g, int nstreams, bool small_blocks, const NoisePlan& plan,
+                    void* buf) {
 	if (fp32) {
 		auto geo = g.template make<float>((float*)out);
 		if (sem == ARMA_NOISE_DOUBLE)
 			launch_streams<float, ARMA_NOISE_DOUBLE>(ctx, hparams, dparams, dseeds, geo, nstreams,
-			                                         small_blocks);
+			                                         small_blocks, plan, buf);
 		else
 			launch_streams<float, ARMA_NOISE_FLOAT>(ctx, hparams, dparams, dseeds, geo, nstreams,
-			                                        small_blocks);
+			                                        small_blocks, plan, buf);
 	} else {
 		auto geo = g.template make<double>((double*)out);
 		if (sem == ARMA_NOISE_DOUBLE)
 			launch_streams<double, ARMA_NOISE_DOUBLE>(ctx, hparams, dparams, dseeds, geo,
-			                                          nstreams, small_blocks);
+			                                          nstreams, small_blocks, plan, buf);
 		else
 			launch_streams<double, ARMA_NOISE_FLOAT>(ctx, hparams, dparams, dseeds, geo,
-			                                         nstreams, small_blocks);
+			                                         nstreams, small_blocks, plan, buf);
 	}
 }
 
@@ -942,7 +1638,16 @@ void launch_white_noise(arma_hip_ctx* ctx, const arma_ar_desc* d, void* eps) {
 	const bool small_blocks = (long long)g.part.x * g.part.y * g.part.z < (1ll << 31);
 	KernelTimer timer(ctx, d->noise_mode == ARMA_NOISE_SEQUENTIAL ? "noise_sequential"
 	                                                               : "noise_partitioned");
-	launch_by_type(ctx, fp32, sem, d->mts, dparams, dseeds, eps, g, ntotal, small_blocks);
+	// (not within a borrowed region, whose size callers reckon without it)
+	NoisePlan plan;
+	if (!ctx->borrow_base)
+		plan = plan_noise(ctx, sem, ntotal,
+		                  (long long)std::min(g.part.x, g.shape.x) *
+		                      std::min(g.part.y, g.shape.y) * std::min(g.part.z, g.shape.z),
+		                  d->mts, small_blocks);
+	void* buf = plan.bytes(ntotal) ? ctx->noise_tmp.get(plan.bytes(ntotal)) : nullptr;
+	launch_by_type(ctx, fp32, sem, d->mts, dparams, dseeds, eps, g, ntotal, small_blocks, plan,
+	               buf);
 }
 
 size_t white_noise_work_bytes(const arma_ar_desc* d) {
@@ -979,8 +1684,9 @@ struct NoiseBatch {
 	int sem = ARMA_NOISE_DOUBLE;
 	int nstreams = 0;
 	bool small_blocks = true;
+	NoisePlan plan;
 	std::vector<arma_mt_params> hparams;
-	Scratch params, seeds, recs;
+	Scratch params, seeds, recs, parts;
 };
 
 NoiseBatch* noise_batch_create(arma_hip_ctx* ctx, int precision,
@@ -1052,6 +1758,12 @@ void noise_batch_build(arma_hip_ctx* ctx, NoiseBatch* b, int precision,
 			}
 		}
 		b->nstreams = int(recs.size());
+		long long longest = 0;
+		for (const NoiseBlockRec& r : recs)
+			longest = std::max(longest, (long long)r.e0 * r.e1 * r.e2);
+		b->plan = plan_noise(ctx, b->sem, b->nstreams, longest, b->hparams.data(),
+		                     b->small_blocks);
+		if (b->plan.bytes(b->nstreams)) b->parts.get(b->plan.bytes(b->nstreams));
 		b->params.get(sizeof(arma_mt_params) * recs.size());
 		b->seeds.get(sizeof(uint32_t) * recs.size());
 		b->recs.get(sizeof(NoiseBlockRec) * recs.size());
@@ -1066,7 +1778,7 @@ void noise_batch_launch(arma_hip_ctx* ctx, NoiseBatch* b, void* arena) {
 	TableSpec g{(const NoiseBlockRec*)b->recs.ptr};
 	launch_by_type(ctx, b->precision == ARMA_FP32, b->sem, b->hparams.data(),
 	               (const arma_mt_params*)b->params.ptr, (const uint32_t*)b->seeds.ptr, arena, g,
-	               b->nstreams, b->small_blocks);
+	               b->nstreams, b->small_blocks, b->plan, b->parts.ptr);
 }
 
 void noise_batch_destroy(NoiseBatch* b) { delete b; }
