@@ -1411,11 +1411,13 @@ SegmentPlan plan_segments(const arma_hip_ctx* ctx, int sem, int nstreams, long l
 
 // Streams of large states take their words from noise_words_kernel when they
 // have at least kAheadNormals normals (below, the extra launches cost what the
-// stream does) and all words fit kAheadBytes.
-constexpr long long kAheadNormals = 8192, kAheadBytes = 256ll << 20;
+// stream does) and all words fit kAheadBytes, or in a batch, whose requests a
+// server admits by bytes that do not count them, kBatchAheadBytes.
+constexpr long long kAheadNormals = 8192, kAheadBytes = 256ll << 20,
+                    kBatchAheadBytes = 16ll << 20;
 
 WordPlan plan_ahead(const arma_hip_ctx* ctx, int sem, int nstreams, long long n,
-                    const arma_mt_params* mts, bool small_blocks) {
+                    const arma_mt_params* mts, bool small_blocks, long long most) {
 	WordPlan wp;
 	int nn_max = 0;
 	for (int i = 0; i < nstreams; ++i) nn_max = std::max(nn_max, int(mts[i].nn));
@@ -1426,7 +1428,7 @@ WordPlan plan_ahead(const arma_hip_ctx* ctx, int sem, int nstreams, long long n,
 	// 4 / pi attempts per pair on average, in whole blocks
 	const long long blocks = (n * 41722 / 65536 + kBlockAttempts) / kBlockAttempts;
 	const long long words = blocks * kBlockAttempts * wpa;
-	if (words * 4 * nstreams > kAheadBytes || blocks > 65535) return wp;
+	if (words * 4 * nstreams > most || blocks > 65535) return wp;
 	wp.words = int(words);
 	wp.blocks = int(blocks);
 	return wp;
@@ -1448,9 +1450,9 @@ struct NoisePlan {
 };
 
 NoisePlan plan_noise(const arma_hip_ctx* ctx, int sem, int nstreams, long long n,
-                     const arma_mt_params* mts, bool small_blocks) {
+                     const arma_mt_params* mts, bool small_blocks, long long ahead_bytes) {
 	NoisePlan plan;
-	plan.ahead = plan_ahead(ctx, sem, nstreams, n, mts, small_blocks);
+	plan.ahead = plan_ahead(ctx, sem, nstreams, n, mts, small_blocks, ahead_bytes);
 	if (plan.ahead.words == 0)
 		plan.seg = plan_segments(ctx, sem, nstreams, n, mts, small_blocks);
 	return plan;
@@ -1644,7 +1646,7 @@ void launch_white_noise(arma_hip_ctx* ctx, const arma_ar_desc* d, void* eps) {
 		plan = plan_noise(ctx, sem, ntotal,
 		                  (long long)std::min(g.part.x, g.shape.x) *
 		                      std::min(g.part.y, g.shape.y) * std::min(g.part.z, g.shape.z),
-		                  d->mts, small_blocks);
+		                  d->mts, small_blocks, kAheadBytes);
 	void* buf = plan.bytes(ntotal) ? ctx->noise_tmp.get(plan.bytes(ntotal)) : nullptr;
 	launch_by_type(ctx, fp32, sem, d->mts, dparams, dseeds, eps, g, ntotal, small_blocks, plan,
 	               buf);
@@ -1762,7 +1764,7 @@ void noise_batch_build(arma_hip_ctx* ctx, NoiseBatch* b, int precision,
 		for (const NoiseBlockRec& r : recs)
 			longest = std::max(longest, (long long)r.e0 * r.e1 * r.e2);
 		b->plan = plan_noise(ctx, b->sem, b->nstreams, longest, b->hparams.data(),
-		                     b->small_blocks);
+		                     b->small_blocks, kBatchAheadBytes);
 		if (b->plan.bytes(b->nstreams)) b->parts.get(b->plan.bytes(b->nstreams));
 		b->params.get(sizeof(arma_mt_params) * recs.size());
 		b->seeds.get(sizeof(uint32_t) * recs.size());
