@@ -1,0 +1,10 @@
+// Batch wavefront kernels, double: many surfaces in one persistent launch.
+#include "ar_batch_kernels.hpp"
+
+namespace arma_hip {
+
+const void* ar_batch_kernel_f64(int tile_x, bool buf, bool dense) {
+	return batch_kernel_by_tile<double, false>(tile_x, buf, dense);
+}
+
+}  // namespace arma_hip

@@ -372,8 +372,8 @@ void arma_hip_partition_shape(const int32_t partition[3], const int32_t grid[3],
 
 enum arma_batch_schedule {
 	ARMA_BATCH_AUTO = 0,
-	ARMA_BATCH_SURFACE_MAJOR = 1,  /* surfaces by decreasing work, tile rows in order */
-	ARMA_BATCH_INTERLEAVED = 2     /* tile rows dealt round-robin over the surfaces */
+	ARMA_BATCH_SURFACE_MAJOR = 1,  /* surfaces by decreasing length of their longest chain */
+	ARMA_BATCH_INTERLEAVED = 2     /* the tiles that can start together, surface by surface */
 };
 
 typedef struct arma_batch_config {
