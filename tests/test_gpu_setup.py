@@ -51,3 +51,32 @@ def test_choi_many_failure_is_per_model(hip_ctx):
     assert res[1] is None
     np.testing.assert_array_equal(res[0][0], hip_ctx.yule_walker_choi(good, 7)[0])
     np.testing.assert_array_equal(res[2][0], hip_ctx.yule_walker_choi(good, 5)[0])
+
+
+@pytest.mark.parametrize("n,order", [
+    (6, 2), (6, 3),     # one panel of the LU, two
+    (10, 6), (10, 9),   # several; factors of more than 256 columns
+    (12, 10), (13, 12),  # matrices of more than 320 rows
+])
+def test_choi_sizes_equal_host(hip_ctx, n, order):
+    """A smooth ACF, and noise in its place, whose matrices pivot in every step:
+    the host solver's result to the last bit, the recursion's stop included."""
+    smooth = O.acf(O.STANDING, (n, n, n), velocity=0.8, beta=(0.8, 0.8))
+    noise = np.random.default_rng(n * 100 + order).standard_normal((n, n, n))
+    noise[0, 0, 0] = 1.0
+    coarse = np.round(2 * noise) / 2  # equal magnitudes: the first largest is the pivot
+    coarse[0, 0, 0] = 1.0
+    holed = smooth.copy()
+    holed[1, 1, 2] = np.nan
+    for acf in (smooth, noise, coarse, holed):
+        for determine in (True, False):
+            try:
+                ref = _abi.yule_walker_choi(acf, order, determine_order=determine)
+            except _abi.ArmaHipError:
+                with pytest.raises(_abi.ArmaHipError):
+                    hip_ctx.yule_walker_choi(acf, order, determine_order=determine)
+                continue
+            got = hip_ctx.yule_walker_choi(acf, order, determine_order=determine)
+            assert got[0].shape == ref[0].shape
+            np.testing.assert_array_equal(got[0], ref[0])
+            assert got[1] == ref[1] or (np.isnan(got[1]) and np.isnan(ref[1]))
