@@ -66,12 +66,14 @@ int ilog2_exact(int n) {
 	return (1 << l) == n ? l : -1;
 }
 
-__global__ void twiddle_kernel(double2* tw, int n) {
-	const int q = blockIdx.x * blockDim.x + threadIdx.x;
-	if (q < n) {
+// e^{-2 pi i q / nx}, q < nx, then e^{-2 pi i q / ny}, q < ny
+__global__ void twiddle_kernel(double2* tw, int nx, int ny) {
+	const int e = blockIdx.x * blockDim.x + threadIdx.x;
+	if (e < nx + ny) {
+		const int q = e < nx ? e : e - nx, n = e < nx ? nx : ny;
 		double s, c;
 		sincospi(2.0 * double(q) / double(n), &s, &c);
-		tw[q] = make_double2(c, -s);  // e^{-2 pi i q / n}
+		tw[e] = make_double2(c, -s);
 	}
 }
 
@@ -373,13 +375,43 @@ struct Summary {
 	Ev second;         // representative of run 2 (complete when runs > 2)
 	Ev prev_last;      // representative of run runs-1
 	Ev last;           // representative of the last run
-	double kmin, kmax; // pairs of adjacent closed runs inside the chunk (3..runs-1)
+	// distances |p1 - p2| of the periods of adjacent closed runs inside the chunk
+	// (3..runs-1): the smallest and the largest
+	double dmin, dmax;
 };
 
-__device__ __forceinline__ double pair_k(const Ev& e1, const Ev& e2) {
-	const double w = kTwoPi / fabs((e1.period - e2.period) * 2.0);
+// The wave number of two adjacent runs at a distance d of their periods.  Every
+// operation rounds monotonically, so the smallest wave number is that of the
+// largest distance, to the bit, and only the two extreme distances need the two
+// divisions.  NaN distances (fmin and fmax pass over them) give NaN wave numbers.
+__device__ __forceinline__ double pair_k(double d) {
+	const double w = kTwoPi / (d * 2.0);
 	return w * w / 9.82;
 }
+
+__device__ __forceinline__ double distance(const Ev& e1, const Ev& e2) {
+	return fabs(e1.period - e2.period);
+}
+
+// Division by one divisor d of ordinary size, y = 1 / d rounded: two remainder
+// steps (Markstein 1990: the first makes the quotient faithful, the second rounds
+// it correctly) in place of the general division's scaling.  Numerators whose
+// remainder could leave the range take the general one.
+struct Divisor {
+	double d, y;
+	bool ordinary;
+	__device__ explicit Divisor(double v)
+	    : d(v), y(1.0 / v), ordinary(fabs(v) > 1e-30 && fabs(v) < 1e30) {}
+	__device__ __forceinline__ bool takes(double x) const {
+		const double m = fabs(x);
+		return m > 1e-200 && m < 1e200;
+	}
+	__device__ __forceinline__ double of(double x) const {
+		double q = x * y;
+		q = fma(fma(-d, q, x), y, q);
+		return fma(fma(-d, q, x), y, q);
+	}
+};
 
 __device__ __forceinline__ Ev first_max(const Ev& cur, const Ev& e) {
 	return fabs(cur.elev) < fabs(e.elev) ? e : cur;
@@ -403,12 +435,12 @@ __device__ __forceinline__ Summary concat(const Summary& a, const Summary& b) {
 	r.runs = na + nb - (merge ? 1 : 0);
 	r.first_pos = a.first_pos;
 	r.last_pos = b.last_pos;
-	r.kmin = fmin(a.kmin, b.kmin);
-	r.kmax = fmax(a.kmax, b.kmax);
+	r.dmin = fmin(a.dmin, b.dmin);
+	r.dmax = fmax(a.dmax, b.dmax);
 	auto score = [&](double p1, double p2) {
-		const double k = pair_k(Ev{p1, 0.0}, Ev{p2, 0.0});
-		r.kmin = fmin(r.kmin, k);
-		r.kmax = fmax(r.kmax, k);
+		const double d = fabs(p1 - p2);
+		r.dmin = fmin(r.dmin, d);
+		r.dmax = fmax(r.dmax, d);
 	};
 	if (merge) {
 		// runs: a_1 .. a_(na-1), J, b_2 .. b_nb
@@ -495,8 +527,9 @@ __global__ __launch_bounds__(1024) void factor_waves_kernel(const T* __restrict_
 	s.runs = 0;
 	s.first_pos = s.last_pos = 0;
 	s.first = s.second = s.prev_last = s.last = Ev{0, 0};
-	s.kmin = 1.7976931348623157e308;
-	s.kmax = 2.2250738585072014e-308;
+	s.dmin = __builtin_inf();
+	s.dmax = -1.0;  // no pair
+	const Divisor by_dt(dt), by_dt2(dt * dt);
 	Ev cur{0, 0}, prev{0, 0};
 	int cur_pos = 0;
 	// the event test and run update at one position (z1, z0, z2 = a-1, a, a+1)
@@ -504,8 +537,16 @@ __global__ __launch_bounds__(1024) void factor_waves_kernel(const T* __restrict_
 		const double dw1 = z0 - z1;
 		const double dw2 = z0 - z2;
 		if ((dw1 > 0.0) != (dw2 > 0.0)) return;
-		const double aa = -0.5 * (dw1 + dw2) / (dt * dt);
-		const double bb = dw1 / dt - aa * dt * (2.0 * t - 1.0);
+		const double curve = -0.5 * (dw1 + dw2);
+		double aa, slope;
+		if (by_dt.takes(dw1) && by_dt2.takes(curve) && by_dt.ordinary && by_dt2.ordinary) {
+			aa = by_dt2.of(curve);
+			slope = by_dt.of(dw1);
+		} else {
+			aa = curve / (dt * dt);
+			slope = dw1 / dt;
+		}
+		const double bb = slope - aa * dt * (2.0 * t - 1.0);
 		const double cc = z0 - t * dt * (aa * t * dt + bb);
 		const double tex = -0.5 * bb / aa;
 		const Ev e{tex, cc + tex * (bb + aa * tex)};
@@ -525,9 +566,9 @@ __global__ __launch_bounds__(1024) void factor_waves_kernel(const T* __restrict_
 			} else if (s.runs == 2) {
 				s.second = cur;
 			} else {
-				const double k = pair_k(cur, prev);
-				s.kmin = fmin(s.kmin, k);
-				s.kmax = fmax(s.kmax, k);
+				const double d = distance(cur, prev);
+				s.dmin = fmin(s.dmin, d);
+				s.dmax = fmax(s.dmax, d);
 			}
 			prev = cur;
 			cur = e;
@@ -619,12 +660,17 @@ __global__ __launch_bounds__(1024) void factor_waves_kernel(const T* __restrict_
 	}
 	if (threadIdx.x == 0) {
 		const Summary& q = sm[0];
-		double kmin = q.kmin, kmax = q.kmax;
+		double dmin = q.dmin, dmax = q.dmax;
 		// the pair (run 2, run 1), which a summary leaves to its caller
 		if (q.runs >= 3) {
-			const double k = pair_k(q.second, q.first);
-			kmin = fmin(kmin, k);
-			kmax = fmax(kmax, k);
+			const double d = distance(q.second, q.first);
+			dmin = fmin(dmin, d);
+			dmax = fmax(dmax, d);
+		}
+		double kmin = 1.7976931348623157e308, kmax = 2.2250738585072014e-308;
+		if (dmax >= 0.0) {
+			kmin = fmin(kmin, pair_k(dmax));
+			kmax = fmax(kmax, pair_k(dmin));
 		}
 		kout[4 * i + dir] = kmin;
 		kout[4 * i + 2 + dir] = kmax;
@@ -1351,8 +1397,7 @@ void run_potential(arma_hip_ctx* ctx, const arma_pot_desc* d, const T* zeta, T* 
 	// twiddles (FP64, generated on the device)
 	double2* twx = (double2*)ctx->pot_twiddle.get(sizeof(double2) * size_t(p.nx + p.ny));
 	double2* twy = twx + p.nx;
-	twiddle_kernel<<<div_ceil(p.nx, 256), 256, 0, st>>>(twx, p.nx);
-	twiddle_kernel<<<div_ceil(p.ny, 256), 256, 0, st>>>(twy, p.ny);
+	twiddle_kernel<<<div_ceil(p.nx + p.ny, 256), 256, 0, st>>>(twx, p.nx, p.ny);
 	int* didx = (int*)ctx->pot_wn.get(sizeof(int) * 2 * size_t(p.nto));
 	int* dtint = didx + p.nto;
 	std::vector<int> both(idx);
