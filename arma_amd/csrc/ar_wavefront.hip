@@ -306,10 +306,12 @@ void launch_typed(arma_hip_ctx* ctx, const arma_ar_desc* d, T* zeta) {
 	upload(ctx, dbuf, tables.data(), tables.size());
 	unsigned char* fb = (unsigned char*)work_buffer(ctx, ctx->flags, p.flag_bytes);
 	T* mbox = (T*)work_buffer(ctx, ctx->mbox, p.mbox_elems * sizeof(T));
-	reset_progress<<<1, 256, 0, ctx->stream>>>((int*)fb, 256 / int(sizeof(int)));
-	ARMA_HIP_CHECK(hipGetLastError());
 	HaloCheck hc;
 	hc.arm(fb);
+	if (!p.var.buf || hc.word) {  // (behind descriptors the zero word is not read)
+		reset_progress<<<1, 256, 0, ctx->stream>>>((int*)fb, 256 / int(sizeof(int)));
+		ARMA_HIP_CHECK(hipGetLastError());
+	}
 	KernelTimer timer(ctx, "ar_wavefront");
 	fill_mailboxes(ctx->stream, mbox, p.mbox_elems);
 	const size_t lds = tile_lds(sizeof(T), p.kTX, P1, P2, p.var.groups, KAHAN);

@@ -157,12 +157,9 @@ inline void* work_buffer(arma_hip_ctx* ctx, Scratch& s, size_t n) {
 	return ctx->borrow_base + at;
 }
 
-// Host-to-device copy of a small, caller-owned host buffer, complete on return.
-inline void upload(arma_hip_ctx* ctx, void* dst, const void* src, size_t bytes) {
-	if (bytes == 0) return;
-	ARMA_HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
-	ARMA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-}
+// Copies a small, caller-owned host buffer to the device in stream order; the
+// buffer may be changed on return.
+void upload(arma_hip_ctx* ctx, void* dst, const void* src, size_t bytes);
 
 // Records msg as the calling thread's last error (arma_hip_last_error).
 void set_last_error(const char* msg);
