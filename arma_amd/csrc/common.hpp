@@ -91,7 +91,7 @@ struct arma_hip_ctx {
 	arma_hip::Scratch params, seeds, state, phi, partials, flags, noise_tmp, mbox;
 	arma_hip::Scratch pot_spec, pot_mid, pot_wn, pot_twiddle, pot_kmin, pot_field, pot_edge,
 	    zeta_tmp, phi_tmp;
-	arma_hip::Scratch yw;
+	arma_hip::Scratch yw, nit_table;
 	int twiddle_n = 0;
 	// a second stream (default priority) on which the potential's row pass of
 	// one chunk overlaps the column pass of the next, and the events that

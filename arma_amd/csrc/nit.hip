@@ -16,6 +16,14 @@
 // function, so the kernel keeps F(a) and F(b) from the step that set them and
 // evaluates F once per step, with identical results.  The Gauss-Legendre
 // nodes are computed on the host (Newton's method on P_20) and passed in.
+//
+// The evaluations (an exp and an erf, or eleven exps, at each of about 25 steps)
+// are the kernel's time.  Every point starts from the same interval, so its first
+// steps visit the same few midpoints as all others': a launch first evaluates F
+// at the midpoints of the first levels (nit_table_kernel, at most a sixteenth as
+// many as there are points) and the points take those steps by look-up, with
+// the same decisions.  300 x 100 x 150 FP64, error 1e-6: 387 us with 18 levels,
+// 720 without.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -67,27 +75,64 @@ __device__ __forceinline__ double target_cdf(const NitParams& p, double x) {
 	return normal_cdf(x, p.mean, p.sigma) - 2.0 * owen_t(p, (x - p.mean) / p.sigma, p.alpha);
 }
 
+// F at the midpoints of the first levels of the bisection: table[1] at the first,
+// table[2 j] and table[2 j + 1] at those of the lower and upper half of the
+// interval whose midpoint is table[j]'s; table[0] = F(a) and, past the last,
+// F(b).
+__global__ __launch_bounds__(256) void nit_table_kernel(double* __restrict__ table, int size,
+                                                        NitParams p) {
+	const int j = int(blockIdx.x) * 256 + int(threadIdx.x);
+	if (j > size) return;
+	double a = p.a, b = p.b;
+	double c = j == 0 ? a : b;
+	if (j > 0 && j < size) {
+		c = 0.5 * (a + b);
+		for (int bit = 30 - __clz(j); bit >= 0; --bit) {
+			if (j >> bit & 1)
+				a = c;
+			else
+				b = c;
+			c = 0.5 * (a + b);
+		}
+	}
+	table[j] = target_cdf(p, c);
+}
+
 template <class T>
-__global__ __launch_bounds__(256) void nit_kernel(T* __restrict__ data, size_t n, NitParams p) {
+__global__ __launch_bounds__(256) void nit_kernel(T* __restrict__ data, size_t n, NitParams p,
+                                                  const double* __restrict__ table, int size) {
 	const size_t stride = size_t(gridDim.x) * blockDim.x;
 	for (size_t q = size_t(blockIdx.x) * blockDim.x + threadIdx.x; q < n; q += stride) {
 		const double y = normal_cdf(double(data[q]), 0.0, p.stdev);
 		double a = p.a, b = p.b, c, fc;
-		double fa = target_cdf(p, a) - y, fb = target_cdf(p, b) - y;
-		int i = 0;
-		do {
-			c = 0.5 * (a + b);
-			fc = target_cdf(p, c) - y;
+		double fa = (size ? table[0] : target_cdf(p, a)) - y;
+		double fb = (size ? table[size] : target_cdf(p, b)) - y;
+		int i = 0, node = 1;
+		// one step from F(c); whether there is another
+		auto step = [&](double f) {
+			fc = f - y;
 			if (fa * fc < 0.0) {
 				b = c;
 				fb = fc;
-			}
-			if (fb * fc < 0.0) {
+				node = 2 * node;
+			} else if (fb * fc < 0.0) {
 				a = c;
 				fa = fc;
+				node = 2 * node + 1;
 			}
 			++i;
-		} while (i < p.max_iter && (b - a) > p.eps && fabs(fc) > p.eps);
+			return i < p.max_iter && (b - a) > p.eps && fabs(fc) > p.eps;
+		};
+		bool more = true;
+		while (more && node < size) {
+			c = 0.5 * (a + b);
+			more = step(table[node]);
+		}
+		while (more) {
+			node = 0;  // (it is past the table)
+			c = 0.5 * (a + b);
+			more = step(target_cdf(p, c));
+		}
 		data[q] = T(c);
 	}
 }
@@ -135,10 +180,33 @@ void launch_nit_realisation(arma_hip_ctx* ctx, void* zeta, size_t n, int precisi
 	if (n == 0) return;
 	const int grid = int(std::min<size_t>((n + 255) / 256, size_t(1) << 20));
 	KernelTimer t(ctx, "nit_realisation");
+	// levels of the table: a sixteenth of the points at most, 2 MB, and no more
+	// than the bisection can take.  A captured launch shares no buffer with the
+	// context's other calls and evaluates every step
+	int levels = 0;
+	hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+	ARMA_HIP_CHECK(hipStreamIsCapturing(ctx->stream, &cap));
+	if (cap == hipStreamCaptureStatusNone) {
+		double width = p.b - p.a;
+		while (levels < 18 && levels < p.max_iter && width > p.eps && (size_t(32) << levels) <= n) {
+			++levels;
+			width *= 0.5;
+		}
+		if (levels < 4) levels = 0;
+	}
+	const int size = levels ? 1 << levels : 0;
+	double* table = nullptr;
+	if (size) {
+		table = (double*)ctx->nit_table.get(sizeof(double) * (size_t(size) + 1));
+		nit_table_kernel<<<size / 256 + 1, 256, 0, ctx->stream>>>(table, size, p);
+		ARMA_HIP_CHECK(hipGetLastError());
+	}
 	if (precision == ARMA_FP32)
-		nit_kernel<float><<<grid, 256, 0, ctx->stream>>>(static_cast<float*>(zeta), n, p);
+		nit_kernel<float><<<grid, 256, 0, ctx->stream>>>(static_cast<float*>(zeta), n, p, table,
+		                                                  size);
 	else
-		nit_kernel<double><<<grid, 256, 0, ctx->stream>>>(static_cast<double*>(zeta), n, p);
+		nit_kernel<double><<<grid, 256, 0, ctx->stream>>>(static_cast<double*>(zeta), n, p, table,
+		                                                   size);
 	ARMA_HIP_CHECK(hipGetLastError());
 }
 

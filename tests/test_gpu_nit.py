@@ -83,3 +83,18 @@ def test_nit_rejects_bad_parameters(hip_ctx):
         d = arma_amd.nit_desc(arma_amd.NIT_GRAM_CHARLIER, **kw)
         with pytest.raises(ValueError):
             hip_ctx.nit_realisation(z, (2, 2, 2), arma_amd.FP64, 1.0, d)
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+@pytest.mark.parametrize("eps,max_iter", [(1e-6, 100), (1e-2, 100), (1e-9, 7), (1e-12, 200)])
+def test_nit_points_do_not_depend_on_how_many_there_are(hip_ctx, name, eps, max_iter):
+    """The first steps' CDF values are shared by the points of a call, as many as
+    their number allows: a point's root is the same bits in any company, the
+    roots that the interval does not bracket, infinities and NaN included."""
+    data = np.random.default_rng(3).standard_normal((64, 96, 128)) * 2.0
+    data[0, 0, :4] = [np.inf, -np.inf, np.nan, 1e3]
+    whole = run(hip_ctx, data, 1.7, CASES[name], arma_amd.FP64, eps, max_iter)
+    for shape in [(1, 1, 5), (1, 7, 128), (9, 96, 128)]:
+        part = np.ascontiguousarray(data[:shape[0], :shape[1], :shape[2]])
+        got = run(hip_ctx, part, 1.7, CASES[name], arma_amd.FP64, eps, max_iter)
+        np.testing.assert_array_equal(got, whole[:shape[0], :shape[1], :shape[2]])
