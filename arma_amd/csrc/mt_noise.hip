@@ -1121,7 +1121,8 @@ __global__ __launch_bounds__(kPcThreads) void noise_wave_kernel(
 // a correlation of g with the 538 words after a segment's start, so the
 // states double in number per level: from segments 0..m-1 to m..2m-1, g
 // squared in between.  Each 16-lane row twists one segment's 538 words into
-// LDS and correlates them (lane k: state word k, lane 15 also word 16).
+// LDS and correlates them (lane k: state word k, lane 15 also word 16), or, where
+// a level has fewer states than the workgroup rows, its share of g's words.
 // noise_count_kernel then counts what each segment accepts, and
 // noise_wave_kernel writes the normals of all segments side by side, each
 // from the sum of the counts before it.  The words, and so the noise, are
@@ -1143,9 +1144,18 @@ __global__ __launch_bounds__(THREADS) void noise_jump_kernel(
 	constexpr int kRows = THREADS / 16;
 	constexpr int kGroups = THREADS / kJumpWords < 8 ? THREADS / kJumpWords : 8;
 	__shared__ uint32_t win[kRows][kJumpStride];
+	// The large workgroup (few streams, much to jump) keeps the residues of all
+	// powers that a square can have above chi's degree: three barriers a square
+	// instead of 34.  With the rows that share a state it took the noise of a 32^3
+	// FP32 surface in 8 streams from 146 to 104 us; many streams in one-wave
+	// workgroups do not miss the barriers, but would the LDS.
+	constexpr bool kTable = THREADS >= 512;
+	constexpr int kSquareRows = (kJumpDegree - 1) / 2;  // t^522, t^524, ..., t^1040
+	__shared__ uint32_t high[kTable ? kSquareRows : 1][kJumpWords];
 	__shared__ uint32_t shift[32][kJumpWords];  // t^(521 + b) mod chi
 	__shared__ uint32_t sq[2 * kJumpWords + 2];
-	__shared__ uint32_t g[kJumpWords];
+	__shared__ uint32_t g[kJumpWords], next_g[kJumpWords];
+	__shared__ uint32_t part[kRows][kWaveNN + 1];
 	const int tid = threadIdx.x;
 	const int row = tid >> 4, k = tid & 15;
 	const arma_mt_params p = params[blockIdx.x];
@@ -1166,6 +1176,7 @@ __global__ __launch_bounds__(THREADS) void noise_jump_kernel(
 		shift[0][tid] = v;
 		// t^e0, e0 at most 512
 		g[tid] = seg.e0 >> 5 == tid ? 1u << (seg.e0 & 31) : 0u;
+		next_g[tid] = 0;
 	}
 	__syncthreads();
 	for (int b = 1; b < 32; ++b) {
@@ -1176,6 +1187,27 @@ __global__ __launch_bounds__(THREADS) void noise_jump_kernel(
 			shift[b][tid] = v ^ (top ? shift[0][tid] : 0u);
 		}
 		__syncthreads();
+	}
+	if constexpr (kTable) {
+		// t^(521 + b + 32) from t^(521 + b): a word up, the bits past the degree
+		// reduced by shift.  Row r = 16 c + q is t^(521 + 2 q + 1 + 32 c).
+		static_assert(16 * kJumpWords <= THREADS, "a lane per word of 16 rows");
+		const int q = tid / kJumpWords, w = tid % kJumpWords;
+		if (q < 16) high[q][w] = shift[2 * q + 1][w];
+		__syncthreads();
+		for (int r0 = 16; r0 < kSquareRows; r0 += 16) {
+			if (q < 16 && r0 + q < kSquareRows) {
+				const uint32_t* from = high[r0 - 16 + q];
+				const uint32_t v =
+					(from[kJumpWords - 2] >> kJumpTop) | (from[kJumpWords - 1] << (32 - kJumpTop));
+				uint32_t x = w ? from[w - 1] : 0u;
+				if (w == kJumpWords - 1) x &= (1u << kJumpTop) - 1u;
+#pragma unroll
+				for (int b = 0; b < 32; ++b) x ^= shift[b][w] & (0u - ((v >> b) & 1u));
+				high[r0 + q][w] = x;
+			}
+			__syncthreads();
+		}
 	}
 	// g <- g^2 mod chi
 	auto square = [&]() {
@@ -1191,6 +1223,30 @@ __global__ __launch_bounds__(THREADS) void noise_jump_kernel(
 			sq[2 * tid + 1] = spread(g[tid] >> 16);
 		}
 		__syncthreads();
+		if constexpr (kTable) {
+			constexpr int kShare = THREADS / kJumpWords;
+			const int q = tid / kJumpWords, w = tid % kJumpWords;
+			if (q < kShare) {
+				uint32_t x = 0;
+				for (int r = q; r < kSquareRows; r += kShare) {
+					const int bit = kJumpDegree + 1 + 2 * r;
+					x ^= high[r][w] & (0u - ((sq[bit >> 5] >> (bit & 31)) & 1u));
+				}
+				uint32_t low = 0;
+				if (q == 0) {
+					low = sq[w];
+					if (w == kJumpWords - 1) low &= (1u << kJumpTop) - 1u;
+				}
+				atomicXor(&next_g[w], x ^ low);
+			}
+			__syncthreads();
+			if (tid < kJumpWords) {
+				g[tid] = next_g[tid];
+				next_g[tid] = 0;
+			}
+			__syncthreads();
+			return;
+		}
 		// 32 bits at a time from the top (the square has degree at most 1040):
 		// bits 521 + 32c .. 521 + 32c + 31 select rows of shift
 		for (int c = 16; c >= 0; --c) {
@@ -1217,49 +1273,72 @@ __global__ __launch_bounds__(THREADS) void noise_jump_kernel(
 	uint32_t* const mine = win[row];
 	for (int m = 1; m < seg.per_stream; m *= 2) {
 		if (m > 1) square();
-		for (int t0 = m; t0 < min(2 * m, seg.per_stream); t0 += kRows) {
-			const int to = t0 + row;
-			const bool act = to < min(2 * m, seg.per_stream);
-			if (!__any(act)) continue;
-			const uint32_t* const from = st + size_t(act ? to - m : 0) * kWaveNN;
-			Twist521 tw{from[k], from[kWaveNN - 1]};
-			mine[k] = tw.s;
-			if (k == 15) mine[16] = tw.t;
-			for (int w = kWaveNN; w < kJumpWindow; w += kWaveNN) {
-				tw.next(k, p);
-				mine[w + k] = tw.s;
-				if (k == 15) mine[w + 16] = tw.t;
-			}
-			wave_lds_order();
-			// state word k: sum of g_i x_(i+k); word 16 one word behind on lane 15
-			uint32_t acc = 0, acc16 = 0, prev = 0;
-			for (int w = 0; w < kJumpWords; ++w) {
-				const uint32_t gw = __builtin_amdgcn_readfirstlane(g[w]);
-				const uint32_t* x = mine + 32 * w + k;
-				if (w < kJumpWords - 1) {
+		const int end = min(2 * m, seg.per_stream);
+		// a level of few states takes several rows for each, which share the words
+		// of g (all of them twist the window)
+		int split = 1;
+		while (split < 16 && 2 * split * (end - m) <= kRows) split *= 2;
+		for (int t0 = m; t0 < end; t0 += kRows / split) {
+			const int to = t0 + row / split, first = row % split;
+			const bool act = to < end;
+			if (__any(act)) {
+				const uint32_t* const from = st + size_t(act ? to - m : 0) * kWaveNN;
+				Twist521 tw{from[k], from[kWaveNN - 1]};
+				mine[k] = tw.s;
+				if (k == 15) mine[16] = tw.t;
+				for (int w = kWaveNN; w < kJumpWindow; w += kWaveNN) {
+					tw.next(k, p);
+					mine[w + k] = tw.s;
+					if (k == 15) mine[w + 16] = tw.t;
+				}
+				wave_lds_order();
+				// state word k: sum of g_i x_(i+k); word 16 one word behind on lane 15
+				uint32_t acc = 0, acc16 = 0;
+				for (int w = first; w < kJumpWords; w += split) {
+					const uint32_t gw = g[w];
+					const uint32_t* x = mine + 32 * w + k;
+					uint32_t prev = 0;
+					if (w < kJumpWords - 1) {
 #pragma unroll
-					for (int b = 0; b < 32; ++b) {
-						const uint32_t mask = 0u - ((gw >> b) & 1u);
-						acc ^= x[b] & mask;
-						acc16 ^= x[b] & prev;
-						prev = mask;
+						for (int b = 0; b < 32; ++b) {
+							const uint32_t mask = 0u - ((gw >> b) & 1u);
+							acc ^= x[b] & mask;
+							acc16 ^= x[b] & prev;
+							prev = mask;
+						}
+						acc16 ^= x[32] & prev;
+					} else {
+#pragma unroll
+						for (int b = 0; b < kJumpTop; ++b) {
+							const uint32_t mask = 0u - ((gw >> b) & 1u);
+							acc ^= x[b] & mask;
+							acc16 ^= x[b] & prev;
+							prev = mask;
+						}
+						acc16 ^= x[kJumpTop] & prev;
+					}
+				}
+				if (split == 1) {
+					if (act) {
+						st[size_t(to) * kWaveNN + k] = acc;
+						if (k == 15) st[size_t(to) * kWaveNN + 16] = acc16;
 					}
 				} else {
-#pragma unroll
-					for (int b = 0; b < kJumpTop; ++b) {
-						const uint32_t mask = 0u - ((gw >> b) & 1u);
-						acc ^= x[b] & mask;
-						acc16 ^= x[b] & prev;
-						prev = mask;
+					part[row][k] = acc;
+					if (k == 15) part[row][16] = acc16;
+				}
+				wave_lds_order();
+			}
+			if (split > 1) {  // one turn of the loop
+				__syncthreads();
+				if (act && first == 0) {
+					for (int w = k; w < kWaveNN; w += 16) {
+						uint32_t x = 0;
+						for (int r = 0; r < split; ++r) x ^= part[row + r][w];
+						st[size_t(to) * kWaveNN + w] = x;
 					}
-					acc16 ^= x[kJumpTop] & prev;
 				}
 			}
-			if (act) {
-				st[size_t(to) * kWaveNN + k] = acc;
-				if (k == 15) st[size_t(to) * kWaveNN + 16] = acc16;
-			}
-			wave_lds_order();
 		}
 		__syncthreads();  // the level's states are the next level's starts
 	}
