@@ -58,7 +58,6 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr double kTwoPi = 6.283185307179586476925286766559;
-constexpr double kFourPi = 12.566370614359172953850573533118;
 
 int ilog2_exact(int n) {
 	int l = 0;
@@ -689,8 +688,10 @@ __device__ __forceinline__ int rot_index(int j, int n) {
 
 // W at one wave number along nz equally spaced levels z_j = zs + j dz, in
 // the working precision R (FP64, or FP32 as the reference's FP32 build
-// evaluates it): W_j = scale (a_j + c_j), a_j = e^{l z_j},
-// c_j = e^{-l (z_j + 2h)}.
+// evaluates it): W_j / 2 = a_j + c_j, a_j = half e^{l z_j},
+// c_j = half e^{-l (z_j + 2h)}, half = 2 pi / (1 + e^{-2 l h}).  (Halves, and the
+// factor within a and c, as the symmetric part is half the sum of two windows: a
+// level costs two products and a sum per window.)
 template <class R>
 struct WinParts {
 	// exponent below which a_j is taken as zero (e^x under 1e-304 in FP64,
@@ -698,7 +699,7 @@ struct WinParts {
 	// evaluated directly
 	static constexpr double kLow = sizeof(R) == 4 ? -80.0 : -700.0;
 	static constexpr double kDirect = sizeof(R) == 4 ? 60.0 : 600.0;
-	R a, c, rho, irho, scale, l;
+	R a, c, rho, irho, half, l;
 	int jstart;   // a_j = 0 for j < jstart
 	bool direct;  // step too large: evaluate the exponentials directly
 
@@ -711,7 +712,7 @@ struct WinParts {
 		const R u = R(du * px), v = R(dv * py);
 		l = R(kTwoPi) * sqrt(u * u + v * v);
 		const R e2h = exp(R(-2) * l * R(h));
-		scale = R(kFourPi) / (R(1) + e2h);
+		half = R(kTwoPi) / (R(1) + e2h);
 		direct = double(l) * fabs(dz) > kDirect;
 		rho = exp(l * R(dz));
 		irho = R(1) / rho;
@@ -728,28 +729,30 @@ struct WinParts {
 		const bool split = js == 0 && !direct && double(l) * fabs(zs) < kDirect &&
 		                   double(l) * 2.0 * h < kDirect;
 		c = split ? e2h / a : exp(-l * R(zs + 2.0 * h));
+		a *= half;
+		c *= half;
 	}
-	// W_j for j = 0, 1, 2, ... in order
+	// W_j / 2 for j = 0, 1, 2, ... in order
 	__device__ __forceinline__ R next(int j, double zs, double dz, double h) {
 		R av, cv;
 		if (direct) {
 			const R zj = R(zs + dz * j);
-			av = exp(l * zj);
-			cv = exp(-l * (zj + R(2.0 * h)));
+			av = half * exp(l * zj);
+			cv = half * exp(-l * (zj + R(2.0 * h)));
 		} else {
 			av = j < jstart ? R(0) : a;
 			cv = c;
 			if (j >= jstart) a *= rho;
 			c *= irho;
 		}
-		return scale * (av + cv);
+		return av + cv;
 	}
 	// Whether every level from j on takes the recurrence with a_j nonzero,
 	// and W_j then, for j = j0, j0 + 1, ... in order once it does: the same
 	// operations as next, without its per-level tests.
 	__device__ __forceinline__ bool plain_from(int j0) const { return !direct && jstart <= j0; }
 	__device__ __forceinline__ R step() {
-		const R v = scale * (a + c);
+		const R v = a + c;
 		a *= rho;
 		c *= irho;
 		return v;
@@ -760,29 +763,24 @@ struct WinParts {
 // (src/velocity/linear_solver.cc:176-183).  Here W only overflows, where
 // z > 0 and l z is large: above ~708 in FP64, where the reference's FP64
 // expression is non-finite too, and above ~88 in FP32, where the value does
-// not fit the working type (as the reference's FP32 expression).
+// not fit the working type (as the reference's FP32 expression).  w is half a
+// window value.
 template <class T>
-__device__ __forceinline__ double finite_or_zero(double w) {
-	return isfinite(T(w)) ? w : 0.0;
+__device__ __forceinline__ T finite_or_zero(T w) {
+	return isfinite(T(2) * w) ? w : T(0);
 }
 
-// Symmetric and antisymmetric parts of the window at one level from
-// W_rot(k) = va and W_rot(-k) = vb.  CHECKED (a level range where W may
-// exceed the working type): non-finite values become zero first and the
-// halves are added (the sum of two values near the top of the range would
-// overflow).  Otherwise 0.5 (va +- vb): the same bits for any pair of
-// values below the top of the range.
-template <class T, bool CHECKED>
-__device__ __forceinline__ void win_pair(double va, double vb, T& w, T& wd) {
+// Symmetric and (ANTI) antisymmetric parts of the window at one level from
+// va = W_rot(k) / 2 and vb = W_rot(-k) / 2.  CHECKED (a level range where W may
+// exceed the working type): non-finite values become zero first.
+template <class T, bool CHECKED, bool ANTI>
+__device__ __forceinline__ void win_pair(T va, T vb, T& w, T& wd) {
 	if constexpr (CHECKED) {
-		va = finite_or_zero<T>(va);
-		vb = finite_or_zero<T>(vb);
-		w = T(0.5 * va + 0.5 * vb);
-		wd = T(0.5 * va - 0.5 * vb);
-	} else {
-		w = T(0.5 * (va + vb));
-		wd = T(0.5 * (va - vb));
+		va = finite_or_zero(va);
+		vb = finite_or_zero(vb);
 	}
+	w = va + vb;
+	wd = ANTI ? va - vb : T(0);
 }
 
 // Whether W may exceed the working type at some level z in [zlo, zhi]:
@@ -856,6 +854,12 @@ __device__ __forceinline__ void col_task(lds_cpx<T>* X, int ny, int M, int nz, i
 		const double zseed = z0 + dz * jseed;
 		// the same for the whole workgroup: one code path per level group
 		const bool checked = window_may_overflow<T>(lmax, zs, zs + dz * (zb - 1));
+		auto by_flags = [&](auto f) {
+			if (checked)
+				ha ? f(std::true_type{}, std::true_type{}) : f(std::true_type{}, std::false_type{});
+			else
+				ha ? f(std::false_type{}, std::true_type{}) : f(std::false_type{}, std::false_type{});
+		};
 		// F * W_sym for the levels of this group
 #pragma unroll
 		for (int e = 0; e < EPT; ++e) {
@@ -874,36 +878,33 @@ __device__ __forceinline__ void col_task(lds_cpx<T>* X, int ny, int M, int nz, i
 						        zseed, dz, h, span);
 					}
 					const int jz = j0 - jseed;
-					auto put = [&](int zz, T w, T wd) {
-						if (ha)
+					auto put = [&](auto ha, int zz, T w, T wd) {
+						if constexpr (ha.value)
 							dst[zz * CB * N] =
 								cpx<T>{f0[e].x * w - g0[e].y * wd, f0[e].y * w + g0[e].x * wd};
 						else
 							dst[zz * CB * N] = cpx<T>{f0[e].x * w, f0[e].y * w};
 					};
-					auto levels = [&](auto checked) {
+					auto levels = [&](auto checked, auto ha) {
 						// the usual case, decided per wave: both windows step by
 						// the plain recurrence at every level of the group
 						if (__all(wa.plain_from(jz) && wb.plain_from(jz))) {
 							for (int zz = 0; zz < zb; ++zz) {
 								T w, wd;
-								win_pair<T, decltype(checked)::value>(wa.step(), wb.step(), w, wd);
-								put(zz, w, wd);
+								win_pair<T, checked.value, ha.value>(wa.step(), wb.step(), w, wd);
+								put(ha, zz, w, wd);
 							}
 							return;
 						}
 						for (int zz = 0; zz < zb; ++zz) {
 							T w, wd;
-							win_pair<T, decltype(checked)::value>(
+							win_pair<T, checked.value, ha.value>(
 								wa.next(jz + zz, zseed, dz, h), wb.next(jz + zz, zseed, dz, h), w,
 								wd);
-							put(zz, w, wd);
+							put(ha, zz, w, wd);
 						}
 					};
-					if (checked)
-						levels(std::true_type{});
-					else
-						levels(std::false_type{});
+					by_flags(levels);
 				}
 				if (ky == 0) {
 					// packed column: add i * F(kx, M) W_sym(kx, M); its window is
@@ -917,14 +918,14 @@ __device__ __forceinline__ void col_task(lds_cpx<T>* X, int ny, int M, int nz, i
 						pa.next(zz, zseed, dz, h);
 						pb.next(zz, zseed, dz, h);
 					}
-					auto levels = [&](auto checked) {
+					auto levels = [&](auto checked, auto ha) {
 						for (int zz = 0; zz < zb; ++zz) {
 							T w, wd;
-							win_pair<T, decltype(checked)::value>(
+							win_pair<T, checked.value, ha.value>(
 								pa.next(jz + zz, zseed, dz, h), pb.next(jz + zz, zseed, dz, h), w,
 								wd);
 							const cpx<T> a = dst[zz * CB * N];
-							if (ha) {
+							if constexpr (ha.value) {
 								const cpx<T> hm{f1[e].x * w - g1[e].y * wd,
 								                f1[e].y * w + g1[e].x * wd};
 								dst[zz * CB * N] = cpx<T>{a.x - hm.y, a.y + hm.x};
@@ -933,10 +934,7 @@ __device__ __forceinline__ void col_task(lds_cpx<T>* X, int ny, int M, int nz, i
 							}
 						}
 					};
-					if (checked)
-						levels(std::true_type{});
-					else
-						levels(std::false_type{});
+					by_flags(levels);
 				}
 			}
 		}
