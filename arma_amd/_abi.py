@@ -608,8 +608,8 @@ class Context:
 
     def yule_walker_choi_many(self, acfs, max_orders, var_eps=1e-6, determine_order=True,
                               chop=True, chop_eps=1e-10):
-        """Choi coefficients of several models in one GPU launch (one
-        workgroup per model): a list of (phi, solver variance), or None for a
+        """Choi coefficients of several models, solved side by side on the
+        GPU: a list of (phi, solver variance), or None for a
         model whose recursion failed."""
         cubes = [np.ascontiguousarray(a, np.float64) for a in acfs]
         ns = np.array([c.shape[0] for c in cubes], np.int32)

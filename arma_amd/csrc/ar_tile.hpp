@@ -34,8 +34,8 @@
 // is not on that chain is moved off it, and the FMAs go to twice the waves.
 // 1024 x 256 x 256 FP64, phi (7, 7, 2): 2.15 ms with one lane per column, all
 // FMAs on the chain, coefficients streamed through the scalar cache and progress
-// counters polled at every step, 0.83 ms so; phi (7, 7, 7) 3.87 and 2.77 ms;
-// 512^3 FP32 (7, 7, 2) 2.5 and 1.08 ms.
+// counters polled at every step, 0.83 ms so; phi (7, 7, 7) 3.87 and 2.73 ms;
+// 512^3 FP32 (7, 7, 7), tiles started in rows and by X + Y, 4.06 and 2.71 ms.
 #pragma once
 
 #include "common.hpp"
@@ -922,7 +922,7 @@ struct BatchSurface {
 	int nY;      // tiles along y
 	int coff;    // coefficient block (elements): the nearest terms, then the bulk's
 	int toff;    // offset table (ints)
-	int poff;    // first progress counter (tiles)
+	int poff;    // first progress counter (the quad tile's)
 	int NB, total_steps;
 	int t0;  // leading slices that are given, not generated
 	int pad;

@@ -186,7 +186,7 @@ void noalloc_setup(int device);
 void yule_walker_choi_device(arma_hip_ctx* ctx, const double* acf, int n, int max_order,
                              double var_eps, bool determine, std::vector<double>& phi, int& l,
                              double& varwn);
-// Several Choi recursions in one launch (one workgroup per model).
+// Several Choi recursions side by side in one sequence of launches.
 struct YwProblem {
 	const double* acf;  // n^3 cube
 	int n, max_order;
@@ -285,8 +285,8 @@ void ar_batch_build(arma_hip_ctx* ctx, ArBatch* b, int precision,
 RescaleBatch* rescale_batch_new();
 void rescale_batch_build(arma_hip_ctx* ctx, RescaleBatch* b, int precision,
                          const std::vector<BatchMember>& m);
-// Device bytes a member adds to a recurrence launch (mailboxes, sink,
-// progress counters).
+// Device bytes a member adds to a recurrence launch (mailboxes, sink;
+// the quad tile's progress counters).
 size_t ar_batch_member_bytes(const arma_ar_desc* d, int tile_x);
 void launch_linear_potential(arma_hip_ctx* ctx, const arma_pot_desc* d, const void* zeta,
                              void* phi, double* wnmax_out);

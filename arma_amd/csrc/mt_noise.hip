@@ -1111,10 +1111,10 @@ __global__ __launch_bounds__(kPcThreads) void noise_wave_kernel(
 // With few streams the launch time of noise_wave_kernel is the length of one
 // stream (29 ns per normal: a twist is a dependent chain), whatever the GPU
 // could do beside it: 2.12 ms for streams of 73728 normals, one or 4096 of
-// them.  Cut in segments, 64 such streams take 0.18 ms, 1000 0.79 ms.  A polar attempt always takes the same number of words,
-// accepted or not, so a stream's words can be cut anywhere between attempts
-// once the generator's state there is known: segment j of a stream starts
-// at its word j L.
+// them.  Cut in segments, 64 such streams take 0.14 ms, 1000 0.79 ms.  A polar
+// attempt always takes the same number of words, accepted or not, so a stream's
+// words can be cut anywhere between attempts once the generator's state there is
+// known: segment j of a stream starts at its word j L.
 //
 // noise_jump_kernel finds those states, one workgroup per stream.  With the
 // residue g = t^(mL) mod chi (mt_jump.hpp) the state m segments further on is

@@ -152,7 +152,7 @@ int arma_hip_ar_generate(arma_hip_ctx* ctx, const arma_ar_desc* desc, void* zeta
    memory (tight serving loops, harnesses that forbid hipMalloc):
    arma_hip_ar_generate with a device pointer zeta and algorithm
    ARMA_AR_WAVEFRONT, whose working buffers (MT records and seeds,
-   coefficient tables, tile progress counters, halo mailboxes) come from a
+   coefficient tables, halo mailboxes) come from a
    static device array of 32 MiB per GPU instead of allocations.  Returns
    ARMA_HIP_EINVAL, before enqueuing anything, for a surface whose buffers
    exceed that (the mailboxes grow with tiles x (nt + 30 + order) x halo
@@ -324,7 +324,7 @@ int arma_hip_yule_walker_choi_device(arma_hip_ctx* ctx, const double* acf, int32
 int arma_hip_white_noise_variance_device(arma_hip_ctx* ctx, const double* acf,
                                          const int32_t acf_shape[3], const double* phi,
                                          const int32_t phi_shape[3], double* out);
-/* Many Choi solves in one launch, one workgroup per model (the models of a
+/* Many Choi solves side by side in one sequence of launches (the models of a
    batch of surfaces; each result equals the single solve's to the last
    bit).  Model i reads the n[i]^3 cube at acf + acf_off[i] and writes at
    most max_order[i]^3 doubles at phi_out + phi_off[i]; order_out[3i..3i+2]
