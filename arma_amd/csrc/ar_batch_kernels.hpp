@@ -81,8 +81,9 @@ __global__ __launch_bounds__(kThreads * G, G == 1 ? 1 : DENSE ? 4 : 2) void ar_b
 	}
 }
 
+// (the dense kernels are a translation unit of their own)
 template <class T, bool KAHAN>
-const void* batch_kernel_by_tile(int tile_x, bool buf, bool dense) {
+const void* batch_kernel_by_tile(int tile_x, bool buf) {
 	auto fn = [](auto* k) { return reinterpret_cast<const void*>(k); };
 	if (tile_x == 8)
 		return buf ? fn(&ar_batch_kernel<T, 8, KAHAN, 1, true, false>)
@@ -90,10 +91,13 @@ const void* batch_kernel_by_tile(int tile_x, bool buf, bool dense) {
 	if (tile_x == 32)
 		return buf ? fn(&ar_batch_kernel<T, 32, KAHAN, 1, true, false>)
 		           : fn(&ar_batch_kernel<T, 32, KAHAN, 1, false, false>);
-	if (!buf) return fn(&ar_batch_kernel<T, 16, KAHAN, 1, false, false>);
-	return dense ? fn(&ar_batch_kernel<T, 16, KAHAN, 2, true, true>)
-	             : fn(&ar_batch_kernel<T, 16, KAHAN, 2, true, false>);
+	return buf ? fn(&ar_batch_kernel<T, 16, KAHAN, 2, true, false>)
+	           : fn(&ar_batch_kernel<T, 16, KAHAN, 1, false, false>);
 }
 
 }  // namespace
+
+const void* ar_batch_dense_f32();
+const void* ar_batch_dense_f64();
+
 }  // namespace arma_hip
