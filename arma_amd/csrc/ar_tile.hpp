@@ -248,9 +248,13 @@ __host__ __device__ constexpr int padded_taps(int p12, int ntr, int chunk) {
 	return p12 <= ntr ? ntr : ntr + (p12 - ntr + chunk - 1) / chunk * chunk;
 }
 // Planes of the LDS ring: the farthest tap of a step was completed
-// P1 + P2 - 3 steps before it; a multiple of the prefetch distance.
+// P1 + P2 - 3 steps before it.  Of two columns a multiple of the prefetch
+// distance, as the steady steps are unrolled over the planes; not otherwise: with
+// FP64 orders of 9 x 10 the planes between would not fit beside the line of an 8 x 32
+// tile.
 __host__ __device__ constexpr int ring_planes(int P1, int P2) {
-	return (P1 + P2 - 2 > 2 ? P1 + P2 - 2 + kD - 1 : kD) / kD * kD;
+	const int n = P1 + P2 - 2 > 2 ? P1 + P2 - 2 : 2;
+	return P2 == 2 ? (n + kD - 1) / kD * kD : n;
 }
 // Row pitch of a plane, in elements.  A wave reads a tap from four rows of 16
 // lanes; in FP32 a pitch of 48 keeps the rows in separate banks where the tight

@@ -123,11 +123,24 @@ void append_tables(const double* phi, int P0, int P1, int P2, int P0S, int group
 }
 
 // LDS bytes of a one-lane tile: the ring, the line and the hand-over.
-size_t tile_lds(int es, int TX, int P1, int P2, int G, bool kahan) {
+constexpr size_t tile_lds(int es, int TX, int P1, int P2, int G, bool kahan) {
 	const int TY = kThreads / TX;
 	return size_t(es) * (size_t(ring_planes(P1, P2)) * (TX + P1 - 1) * ring_pitch(es, TX, P1, P2, G) +
 	                     size_t(TY + 1) * kThreads + (G > 1 ? 2 * kThreads * (kahan ? 2 : 1) : 0));
 }
+
+// Every order whose halo a tile's width admits (ar_batch_fits) has its LDS, beside
+// the kernel's own few words: nothing else decides what a batch takes.
+constexpr bool all_orders_fit() {
+	for (int es : {4, 8})
+		for (int TX : {8, 16, 32})
+			for (int P1 = 1; P1 <= kMaxP12 && P1 - 1 <= TX; ++P1)
+				for (int P2 = 1; P2 <= kMaxP12 && P2 - 1 <= kThreads / TX; ++P2)
+					for (int G = 1; G <= (TX == 16 ? 2 : 1); ++G)
+						if (tile_lds(es, TX, P1, P2, G, es == 4) + 256 > 160 * 1024) return false;
+	return true;
+}
+static_assert(all_orders_fit(), "an order's LDS exceeds the CU's");
 
 // Whether a surface's accesses go through buffer descriptors: the mailboxes
 // from a tile's corner neighbour to itself, and the slices of a step's noise
