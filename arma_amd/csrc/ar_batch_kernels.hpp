@@ -1,6 +1,6 @@
 // The batch kernel of the one-lane wavefront tile.  DENSE: two workgroups per
-// CU, for batches whose known shapes all fit kDenseRegs (5 FP32 surfaces of
-// orders up to 5: 513 us against 690 with one).
+// CU, for batches whose known shapes all fit kDenseRegs (15 FP32 surfaces of
+// orders up to 5: 490 us against 635 with one).
 #pragma once
 
 #include "ar_tile.hpp"
@@ -53,7 +53,7 @@ __global__ __launch_bounds__(kThreads * G, G == 1 ? 1 : DENSE ? 4 : 2) void ar_b
 	case kBatchBuckets + P - kShapedMin:                                                      \
 		if constexpr (G == 2 && two_columns_fit(sizeof(T), P) &&                              \
 		              (!DENSE || is_dense(sizeof(T), P, kTwoColumns)))                        \
-			ARMA_BATCH_TILE(P, 2 * P, kTwoColumns);                                           \
+			ARMA_BATCH_TILE(P, 2 * P - 1, kTwoColumns);                                           \
 		break;                                                                                \
 	case kBatchBuckets + kShaped + P - kShapedMin:                                            \
 		if constexpr (G == 2 && (!DENSE || is_dense(sizeof(T), P, kSquare)))                  \

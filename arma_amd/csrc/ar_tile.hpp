@@ -10,8 +10,8 @@
 //    in-slice dependency (x-i, y-j) was finished at an earlier step: the skew
 //    replaces the reference's partition DAG inside the tile.
 //  * "Push" form of the sum: each value zeta(t, x-i, y-j) is read once from LDS
-//    and feeds the partial sums of the points (t+k, x, y), k < P0, which the
-//    lane keeps in registers: P1*P2 LDS reads feed P0*P1*P2 FMAs.
+//    by each group and feeds the partial sums of the points (t+k, x, y), k < P0,
+//    which the lanes keep in registers: P1*P2 LDS reads feed P0*P1*P2 FMAs.
 //  * LDS holds a ring of planes, one per step, of the tile plus its causal halo
 //    (P1-1 rows above, P2-1 columns to the left).
 //  * Halo values come from the neighbouring tiles through HBM.  Each tile keeps
@@ -29,13 +29,12 @@
 //    each step adds one P1*P2-term FP32 partial to it.
 //
 // What bounds it: a step is a chain from the last step's values to this one's,
-// write - barrier - read - a few operations - write, about 0.2 us, plus the FMAs
-// of one step (P0*P1*P2 of four cycles per wave and SIMD), so everything that
-// is not on that chain is moved off it, and the FMAs go to twice the waves.
-// 1024 x 256 x 256 FP64, phi (7, 7, 2): 2.15 ms with one lane per column, all
-// FMAs on the chain, coefficients streamed through the scalar cache and progress
-// counters polled at every step, 0.83 ms so; phi (7, 7, 7) 3.87 and 2.73 ms;
-// 512^3 FP32 (7, 7, 7), tiles started in rows and by X + Y, 4.06 and 2.71 ms.
+// write - barrier - read - part[0] - write, about 0.3 us, plus the FMAs of one
+// step (P0*P1*P2 of four cycles per wave and SIMD), which go to twice the waves.
+// 1024 x 256 x 256 FP64, phi (7, 7, 2): 2.16 ms with one lane per column,
+// coefficients streamed through the scalar cache and progress counters polled at
+// every step, 0.84 ms so; phi (7, 7, 7) 3.84 and 2.77 ms; 512^3 FP32 (7, 7, 7) 6.5 and
+// 2.6 ms, 2048 x 512 x 512 FP32 (7, 7, 2) 7.65 and 2.88 ms.
 #pragma once
 
 #include "common.hpp"
@@ -200,37 +199,37 @@ __device__ __forceinline__ int wrap_inc(int v, int r) { return v + 1 == r ? 0 : 
 
 // ---- tables of one surface ----
 //
-// The sum of a point is split by when its terms become known.  At step s a
-// lane completes a point whose neighbours at skew distance 1 (the point
-// before it in t, x or y) were completed at step s - 1; everything else is
-// known a step earlier.  So a step first adds the nearest terms to the
-// sum of everything else (the "critical" part, a few dependent operations),
-// writes the point, and then, while nobody waits for it, adds up everything
-// else of its next point (the "bulk").
+// At step s a lane completes a point of slice t = s - x - y.  By then everything
+// that its neighbours (x - i, y - j), i + j > 0, have of slice t was completed at
+// earlier steps, so the step adds up the slice's part of the sums of all slices
+// t + k, k < P0, before the point itself is known:
+//   part[k] = sum of phi(k, i, j) zeta(t, x - i, y - j), (i, j) != (0, 0)
+// as a chain of FMAs from zero over the taps in row-major order; the point takes
+// acc[0] + part[0], and acc[k] of the others gets part[k] + phi(k, 0, 0) times the
+// point, one addition per slice.  In FP32 that addition is compensated.
 //
-// (The nearest term in t, phi(1,0,0) times the point just completed, goes to the
-// next point's sum by itself, first.)
+// The order is part of the result: fitted coefficients of a standing wave are
+// large and cancel (sum of |phi| 13-20 for a variance of 1), so that sums taken in
+// another order differ by more than the rounding of their results, and a
+// transform of the surface that is flat or not monotone (NIT) makes visible steps
+// of it.  Adding the nearest terms apart from the others leaves only a few
+// operations between the last step's values and a point, 0.79 in place of
+// 0.84 ms above, but came out up to 1.4 times as far from 64 bits in FP32.
 //
-// Bulk, push form: with q the slice of the lane's next point, tap m = (i, j)
-// brings one value V_m from LDS and adds C[r][m] V_m to accumulator r, the
-// partial sum of slice q + r (r < P0).  V_m is slice q where i + j >= 2, q - 1
-// where i + j = 1 and q - 2 where i = j = 0 (the latest values that are in
-// LDS before this step), so C[r][m] = phi(r, i, j), phi(r + 1, i, j) and
-// phi(r + 2, 0, 0) (zero past phi's extent in t).
+// The accumulators may be split between two groups of waves (256 lanes each, the
+// same columns): group 0 has k < K0, the point and the memory traffic, group 1
+// has k >= K0.  Group 1 takes its points a step late, from LDS, and hands slice
+// t + K0 to group 0 through LDS at every step: the sum so far and part[K0], to
+// which group 0, which has the point, adds phi(K0, 0, 0) times it.  The split
+// changes no sum.
 //
-// The accumulators may be split between two groups of waves (256 lanes each,
-// the same columns): group 0 has r < K0, the critical part and the memory
-// traffic, group 1 has r >= K0 and hands its accumulator K0 to group 0's
-// K0 - 1 through LDS every step.  The split changes no sum.
-//
-// Tables: near[0..3] = phi(0,0,0), phi(1,0,0), phi(0,1,0), phi(0,0,1) (zero
-// where phi has no such term), then per group the coefficients [tap][r] of its
-// accumulators, taps in row-major order padded with zero coefficients.
-// Offsets: LDS holds the last R' steps' values of the tile and its halo, one
-// plane per step (step s in plane s mod R'), so a tap's distance is uniform
-// over the tile but turns with the step: row s mod R' of the offset table has
-// the byte offsets of [this step's plane, the x and y neighbours of the
-// critical part, unused, the taps].
+// Tables: near[k] = phi(k, 0, 0), k < P0, then per group the coefficients
+// [tap][k] of its accumulators, taps (0, 1), (0, 2), ... in row-major order padded
+// with zero coefficients.  Offsets: LDS holds the last R steps' values of the tile
+// and its halo, one plane per step (step s in plane s mod R), so a tap's distance
+// is uniform over the tile but turns with the step: row s mod R of the offset
+// table has the byte offsets of [this step's plane, the last step's, unused, unused,
+// the taps].
 
 // The first NTR taps' coefficients (a template parameter) stay in vector
 // registers, the others are streamed through the scalar cache in chunks of
@@ -240,36 +239,36 @@ __host__ __device__ constexpr int chunk_taps(int es, int k) {
 	while (c > 1 && c * k * es > 256) c /= 2;
 	return c;
 }
-constexpr int kNear = 16;  // elements before the coefficients
+constexpr int kNear = 16;  // elements before the coefficients, phi(k, 0, 0) in the first
 constexpr int kOffHead = 4;
 
-// Taps padded to the kernel's units.
-__host__ __device__ constexpr int padded_taps(int p12, int ntr, int chunk) {
-	return p12 <= ntr ? ntr : ntr + (p12 - ntr + chunk - 1) / chunk * chunk;
+// n taps padded to the kernel's units.
+__host__ __device__ constexpr int padded_taps(int n, int ntr, int chunk) {
+	return n <= ntr ? ntr : ntr + (n - ntr + chunk - 1) / chunk * chunk;
 }
 // Planes of the LDS ring: the farthest tap of a step was completed
-// P1 + P2 - 3 steps before it.  Of two columns a multiple of the prefetch
+// P1 + P2 - 2 steps before it.  Of two columns a multiple of the prefetch
 // distance, as the steady steps are unrolled over the planes; not otherwise: with
 // FP64 orders of 9 x 10 the planes between would not fit beside the line of an 8 x 32
 // tile.
 __host__ __device__ constexpr int ring_planes(int P1, int P2) {
-	const int n = P1 + P2 - 2 > 2 ? P1 + P2 - 2 : 2;
+	const int n = P1 + P2 - 1 > 2 ? P1 + P2 - 1 : 2;
 	return P2 == 2 ? (n + kD - 1) / kD * kD : n;
 }
 // Row pitch of a plane, in elements.  A wave reads a tap from four rows of 16
 // lanes; in FP32 a pitch of 48 keeps the rows in separate banks where the tight
-// pitch TY + P2 - 1 does not (1024 x 16 x 16, phi (5, 5, 5): 573 against 496 us,
-// phi (7, 7, 7): 1200 against 962 us).  In FP64 it measured the same as the
+// pitch TY + P2 - 1 does not (1024 x 16 x 16, phi (5, 5, 5): 611 against 529 us,
+// phi (7, 7, 7): 1110 against 935 us).  In FP64 it measured the same as the
 // tight one (1570 against 1557 us), which leaves more LDS.
 __host__ __device__ constexpr int ring_pitch(int es, int TX, int P1, int P2, int groups) {
 	const int TY = kThreads / TX, tight = TY + P2 - 1;
 	if (es != 4 || TX != 16 || groups == 1) return tight;
-	const int rest = (TY + 1) * kThreads * es + 4 * kThreads * es;  // line, hand-over
+	const int rest = (TY + 1) * kThreads * es + 6 * kThreads * es;  // line, hand-over
 	return ring_planes(P1, P2) * (TX + P1 - 1) * 48 * es + rest <= 160 * 1024 ? 48 : tight;
 }
 
-// Accumulators of group 0 of two.  Group 0 also has the critical part and the
-// memory traffic, about 60 instructions a step, so with few taps it takes the
+// Accumulators of group 0 of two.  Group 0 also has the point and the memory
+// traffic, about 60 instructions a step, so with few taps it takes the
 // fewest accumulators that leave group 1's coefficients room in its registers;
 // with many the halves are even.
 constexpr int kCoefRegs = 196;  // 32-bit registers for coefficients, of 256 at two waves per SIMD
@@ -277,28 +276,32 @@ constexpr int kDenseRegs = 84;  // of 128 at four
 __host__ __device__ constexpr int group_split(int es, int p0, TapShape shape) {
 	const int half = p0 > 2 ? (p0 - 1) / 2 : 1;
 	if (shape != kTwoColumns) return half;
-	const int most = 2 * p0 * (p0 - half) * (es / 4) <= kDenseRegs ? kDenseRegs : kCoefRegs;
+	const int most = (2 * p0 - 1) * (p0 - half) * (es / 4) <= kDenseRegs ? kDenseRegs : kCoefRegs;
 	int k = p0 / 4 > 1 ? p0 / 4 : 1;
-	while (k < half && 2 * p0 * (p0 - k) * (es / 4) > most) ++k;
+	while (k < half && (2 * p0 - 1) * (p0 - k) * (es / 4) > most) ++k;
 	return k;
 }
 __host__ __device__ constexpr int group_most(int es, int p0, int groups, TapShape shape) {
 	const int k = group_split(es, p0, shape);
 	return groups == 1 ? p0 : p0 - k > k ? p0 - k : k;
 }
-// Resident taps of the kernels with known shapes.
+// Resident taps of the kernels with known shapes.  Of a square order, as many as
+// leave room for the sums, parts and row offsets of its P0: with more the kernels
+// kept 5 to 80 registers in scratch memory (512 x 256 x 256 FP64, phi (9, 9, 9): 19
+// taps 5.28 ms, 13 3.47 ms; (7, 7, 7): 24 taps 2.28 ms, 19 1.91 ms, 13 2.05 ms).
 __host__ __device__ constexpr bool two_columns_fit(int es, int p0) {
-	return p0 > 1 && 2 * p0 * group_most(es, p0, 2, kTwoColumns) * (es / 4) <= kCoefRegs;
+	return p0 > 1 && (2 * p0 - 1) * group_most(es, p0, 2, kTwoColumns) * (es / 4) <= kCoefRegs;
 }
 __host__ __device__ constexpr int square_taps(int es, int p0) {
-	const int n = kCoefRegs / (group_most(es, p0, 2, kSquare) * (es / 4));
-	return n < p0 * p0 ? n : p0 * p0;
+	const int w = es / 4, n = (238 - 6 * p0 * w) / (group_most(es, p0, 2, kSquare) * w);
+	return n < p0 * p0 - 1 ? n : p0 * p0 - 1;
 }
 // Whether two workgroups of two groups share a CU: all coefficients of a known
 // shape within kDenseRegs, or none resident.
 __host__ __device__ constexpr bool is_dense(int es, int p0, TapShape shape) {
 	return shape == kAnyShape ||
-	       (shape == kTwoColumns ? 2 : p0) * p0 * group_most(es, p0, 2, shape) * (es / 4) <= kDenseRegs;
+	       ((shape == kTwoColumns ? 2 : p0) * p0 - 1) * group_most(es, p0, 2, shape) * (es / 4) <=
+	           kDenseRegs;
 }
 
 // Mailbox column of tile-local lane (x, y), or -1 when no neighbour reads it:
@@ -327,12 +330,10 @@ struct PhaseRow {
 	static __device__ constexpr unsigned at(int steps, int i, int j) {
 		return unsigned((((PH - steps) % R + R) % R * kPlane - i * WY - j) * int(sizeof(T)));
 	}
-	__device__ constexpr unsigned head(int e) const {
-		return e == 0 ? at(0, 0, 0) : e == 1 ? (P0 > 1 ? at(1, 1, 0) : at(0, 0, 0)) : at(1, 0, 1);
-	}
-	__device__ constexpr unsigned tap(int m) const {
-		const int i = m / 2, j = m % 2;
-		return at((i + j > 2 ? i + j : 2) - 1, i, j);
+	__device__ constexpr unsigned head(int e) const { return at(e, 0, 0); }
+	__device__ constexpr unsigned tap(int e) const {
+		const int i = (e + 1) / 2, j = (e + 1) % 2;
+		return at(i + j, i, j);
 	}
 };
 
@@ -390,8 +391,9 @@ __device__ __forceinline__ void wave_tile(
 	static_assert(kTX * kTY == kThreads && kTX >= 8 && kTY >= 8, "tile shape");
 	static_assert(G == 1 || P0 > 1, "two groups need two accumulators");
 	constexpr bool TWO = SH == kTwoColumns, SQ = SH == kSquare;
-	static_assert(!TWO || NTR == 2 * P0, "all taps of a P0 x 2 order are resident");
-	static_assert(!SQ || NTR <= P0 * P0, "no more taps than the order has");
+	static_assert(!TWO || NTR == 2 * P0 - 1, "all taps of a P0 x 2 order are resident");
+	static_assert(!SQ || NTR < P0 * P0, "no more taps than the order has");
+	static_assert(P0 <= kNear, "phi(k, 0, 0) before the coefficients");
 	constexpr int KD = kD;
 	const int P1 = SH == kAnyShape ? P1_ : P0, P2 = TWO ? 2 : SQ ? P0 : P2_;
 	constexpr int kCH = chunk_taps(sizeof(T), group_most(sizeof(T), P0, G, SH));
@@ -410,15 +412,15 @@ __device__ __forceinline__ void wave_tile(
 	const int group = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(thread / kThreads);
 	const int tid = thread % kThreads;
 	const int lx = tid / kTY, ly = tid - (tid / kTY) * kTY;
-	const int ntap = padded_taps(P1 * P2, NTR, kCH);
+	const int ntap = padded_taps(P1 * P2 - 1, NTR, kCH);
 	const int orow = kOffHead + ntap;  // ints per row of the offset table
 
 	// LDS: the ring of planes, a line of kDL slots per lane, and with two
-	// groups the handed-over accumulators of two steps
+	// groups the hand-over of two steps (a part, and the sum that it goes to)
 	unsigned char* const ring = smem_raw;
 	constexpr int kDL = kTY + 1;
 	T* const line = reinterpret_cast<T*>(smem_raw + size_t(R) * plane * sizeof(T)) + tid;
-	using Hand = std::conditional_t<KAHAN, T[2], T[1]>;
+	using Hand = std::conditional_t<KAHAN, T[3], T[2]>;
 	Hand* const hand = reinterpret_cast<Hand*>(line - tid + kDL * kThreads) + tid;
 	const unsigned own = unsigned(((lx + HX) * pitch + (ly + HY)) * sizeof(T));
 	auto lds = [&](unsigned at) -> T& { return *reinterpret_cast<T*>(ring + at); };
@@ -432,7 +434,7 @@ __device__ __forceinline__ void wave_tile(
 	// everything in LDS starts zeroed: halo positions outside the grid, slices
 	// before the first and their noise stay zero
 	{
-		const int words = R * plane + kDL * kThreads + (G > 1 ? 2 * kThreads * (KAHAN ? 2 : 1) : 0);
+		const int words = R * plane + kDL * kThreads + (G > 1 ? 2 * kThreads * (KAHAN ? 3 : 2) : 0);
 		for (int q = thread; q < words; q += G * kThreads) reinterpret_cast<T*>(smem_raw)[q] = T(0);
 	}
 	int ph = s0 % R;  // plane of this step
@@ -442,63 +444,58 @@ __device__ __forceinline__ void wave_tile(
 	// table, read a step ahead into scalar registers (the head and the resident
 	// taps; for a square order the head and one base per distance), or
 	// constants of the phase.
-	constexpr int kFar = 2 * P0 - 2;                   // largest distance of a square order
-	constexpr int kBases = kFar > 2 ? kFar - 1 : 1;    // its distances 2 .. kFar
-	constexpr int kRow = 3 + (SQ ? kBases : NTR);
+	constexpr int kP2 = TWO ? 2 : P0, kW = ring_pitch(sizeof(T), TX, P0, kP2, G);
+	constexpr int kBases = P0 > 1 ? 2 * P0 - 2 : 1;  // distances of a square order's taps
+	constexpr int kRow = 2 + (SQ ? kBases : NTR);
 	struct Row {
 		int o[kRow];
 		__device__ unsigned head(int e) const { return unsigned(o[e]); }
 		__device__ unsigned tap(int m) const {
-			return unsigned(o[SQ ? 0 : 3 + m]);
+			return unsigned(o[SQ ? 0 : 2 + m]);
 		}
 	};
 	auto read_row = [&](int phase, Row& r) {
 		const int* const p = offs + phase * orow;
 #pragma unroll
-		for (int e = 0; e < 3; ++e) r.o[e] = p[e];
+		for (int e = 0; e < 2; ++e) r.o[e] = p[e];
 		if constexpr (SQ) {
 			// tap (0, d) or (d - P0 + 1, P0 - 1) of each distance d, without its
 			// distance within the plane
-			constexpr int kW = ring_pitch(sizeof(T), TX, P0, P0, G);
 #pragma unroll
-			for (int d = 2; d < 2 + kBases; ++d) {
+			for (int d = 1; d <= kBases; ++d) {
 				const int i = d < P0 ? 0 : d - P0 + 1, j = d < P0 ? d : P0 - 1;
-				r.o[3 + d - 2] = P0 > 1 ? p[kOffHead + i * P0 + j] + (i * kW + j) * int(sizeof(T)) : 0;
+				r.o[1 + d] = p[kOffHead + i * P0 + j - 1] + (i * kW + j) * int(sizeof(T));
 			}
 		} else {
 #pragma unroll
-			for (int e = 0; e < NTR; ++e) r.o[3 + e] = p[kOffHead + e];
+			for (int e = 0; e < NTR; ++e) r.o[2 + e] = p[kOffHead + e];
 		}
 	};
 	auto hold_row = [](Row& r) {
 #pragma unroll
 		for (int e = 0; e < kRow; ++e) asm volatile("" : "+s"(r.o[e]));
 	};
-	// a tap's value; the square order's constant offsets, all within own's
-	// distance from the start of its plane, as nonnegative ones from a base
-	auto at_tap = [&](const auto& row, int m) {
+	// a tap's value from base, the farthest in-plane distance before own, so that
+	// a known order's constant offsets are nonnegative
+	constexpr unsigned kBack = SH == kAnyShape ? 0u : unsigned(((P0 - 1) * kW + kP2 - 1) * sizeof(T));
+	auto at_tap = [&](const auto& row, int e, unsigned base) {
 		if constexpr (SQ) {
-			constexpr int kW = ring_pitch(sizeof(T), TX, P0, P0, G);
-			constexpr unsigned kBack = unsigned(((P0 - 1) * kW + P0 - 1) * sizeof(T));
-			const int i = m / P0, j = m % P0;
-			const unsigned base = own - kBack + unsigned(row.o[3 + (i + j > 2 ? i + j - 2 : 0)]);
-			return lds(base + (kBack - unsigned((i * kW + j) * sizeof(T))));
+			const int i = (e + 1) / P0, j = (e + 1) % P0;
+			return lds(base + unsigned(row.o[1 + i + j]) + (kBack - unsigned((i * kW + j) * sizeof(T))));
 		} else {
-			return lds(own + row.tap(m));
+			return lds(base + (kBack + row.tap(e)));
 		}
 	};
-	// the bulk of one group: its K accumulators, with the coefficients cf
-	auto bulk_of = [&](auto kc, const T* __restrict__ cf, auto& creg, auto& acc, int phase,
-	                   const auto& row) {
+	// the parts of one group's K accumulators, with the coefficients cf
+	auto parts_of = [&](auto kc, const T* __restrict__ cf, auto& creg, auto& part, int phase,
+	                    const auto& row) {
 		constexpr int K = decltype(kc)::value;
-		T part[K];
+		// opaque in every step where two workgroups share a CU: the addresses of the
+		// unrolled phases, kept over the loop, did not fit beside the coefficients
+		unsigned base = own - kBack;
+		if constexpr (TWO && is_dense(sizeof(T), P0, SH)) asm volatile("" : "+v"(base));
 #pragma unroll
-		for (int r = 0; r < K; ++r) {
-			if constexpr (KAHAN)
-				part[r] = T(0);
-			else
-				part[r] = acc[r].s;
-		}
+		for (int r = 0; r < K; ++r) part[r] = T(0);
 		if constexpr (NTR > 0) {
 			// the values in runs of 16, so that they do not crowd out the
 			// coefficients
@@ -507,7 +504,7 @@ __device__ __forceinline__ void wave_tile(
 				T v[16];
 #pragma unroll
 				for (int m = 0; m < 16; ++m)
-					if (m0 + m < NTR) v[m] = at_tap(row, m0 + m);
+					if (m0 + m < NTR) v[m] = at_tap(row, m0 + m, base);
 #pragma unroll
 				for (int m = 0; m < 16; ++m)
 					if (m0 + m < NTR) {
@@ -517,34 +514,19 @@ __device__ __forceinline__ void wave_tile(
 					}
 			}
 		}
-		if constexpr (!TWO && !(SQ && NTR == P0 * P0)) {
+		if constexpr (!TWO && !(SQ && NTR == P0 * P0 - 1)) {
 			const int* to = offs + phase * orow + kOffHead + NTR;
 			cf += NTR * K;
 #pragma unroll 1
 			for (int c = NTR; c < ntap; c += kCH, cf += kCH * K, to += kCH) {
 				T v[kCH];
 #pragma unroll
-				for (int m = 0; m < kCH; ++m) {
-					v[m] = lds(own + unsigned(to[m]));
-					// order 1 in t takes nothing from earlier slices, not even zero
-					// times inf
-					if constexpr (P0 == 1) {
-						const int a = c + m, i = a / P2, j = a - i * P2;
-						v[m] = a < P1 * P2 && i + j > 1 ? v[m] : T(0);
-					}
-				}
+				for (int m = 0; m < kCH; ++m) v[m] = lds(own + unsigned(to[m]));
 #pragma unroll
 				for (int m = 0; m < kCH; ++m)
 #pragma unroll
 					for (int r = 0; r < K; ++r) part[r] = fma(cf[m * K + r], v[m], part[r]);
 			}
-		}
-#pragma unroll
-		for (int r = 0; r < K; ++r) {
-			if constexpr (KAHAN)
-				acc[r].add(part[r]);
-			else
-				acc[r].s = part[r];
 		}
 	};
 	// keeps a step's sums in the step: left free, the compiler defers them to
@@ -552,6 +534,8 @@ __device__ __forceinline__ void wave_tile(
 	auto pin = [](auto& acc) {
 		for (auto& a : acc) a.pin();
 	};
+	// phi(k, 0, 0) of accumulator k of the group
+	auto near_of = [&](int k) { return k < P0 ? near[k] : T(0); };
 	// coefficients kept in registers: loaded once, and opaque to the compiler,
 	// which would otherwise keep uniform values in (and spill them from) the
 	// scalar registers
@@ -571,9 +555,14 @@ __device__ __forceinline__ void wave_tile(
 		const T* const cf = coef + ntap * K0;
 		T creg[NTR > 0 ? NTR * KC::value : 1];
 		load_coef(KC{}, cf, creg);
+		T c00[KC::value], part[KC::value];
 		Acc<T, KAHAN> acc[KC::value];
 #pragma unroll
-		for (int r = 0; r < KC::value; ++r) acc[r].zero();
+		for (int r = 0; r < KC::value; ++r) {
+			acc[r].zero();
+			part[r] = T(0);
+			c00[r] = near_of(K0 + r);
+		}
 		Row o;
 		read_row(ph, o);
 		__syncthreads();
@@ -582,15 +571,23 @@ __device__ __forceinline__ void wave_tile(
 			const int pn = wrap_inc(ph, R);
 			Row on;
 			if constexpr (!kConst) read_row(pn, on);
-			// slice q + r of the last step is q + r - 1 of this one
+			// the last step's point completes that step's sums; accumulator r of
+			// this step is r + 1 of the last
+			const T zl = lds(own + row.head(1));
 #pragma unroll
-			for (int r = 0; r + 1 < KC::value; ++r) acc[r] = acc[r + 1];
+			for (int r = 1; r < KC::value; ++r) {
+				acc[r].add(fma(c00[r], zl, part[r]));
+				acc[r - 1] = acc[r];
+			}
 			acc[KC::value - 1].zero();
-			bulk_of(KC{}, cf, creg, acc, ph, row);
-			pin(acc);
 			Hand& h = hand[(u & 1) * kThreads];
-			h[0] = acc[0].s;
-			if constexpr (KAHAN) h[1] = acc[0].c;
+			h[1] = acc[0].s;
+			if constexpr (KAHAN) h[2] = acc[0].c;
+			parts_of(KC{}, cf, creg, part, ph, row);
+			h[0] = part[0];
+			pin(acc);
+#pragma unroll
+			for (int r = 1; r < KC::value; ++r) asm volatile("" : "+v"(part[r]));
 			if constexpr (!kConst) {
 				ph = pn;
 				hold_row(on);
@@ -784,8 +781,11 @@ __device__ __forceinline__ void wave_tile(
 	Acc<T, KAHAN> acc[K0];
 #pragma unroll
 	for (int r = 0; r < K0; ++r) acc[r].zero();
-	const T n000 = near[0], n100 = near[1], n010 = near[2], n001 = near[3];
+	T c00[K0 + 1];
+#pragma unroll
+	for (int r = 0; r < K0 + 1; ++r) c00[r] = near_of(r);
 	T eps = T(0);  // the noise of the lane's next point
+	T zl = T(0);   // its last point
 	// line slots: this step's (the noise arriving, the value leaving), the next
 	// point's, and this point's
 	int dl = s0 % kDL, dn = (s0 - ly) % kDL, dw = (s0 - ly - 1) % kDL;
@@ -808,28 +808,20 @@ __device__ __forceinline__ void wave_tile(
 		Row on;
 		if constexpr (!kConst) read_row(pn, on);
 		const unsigned here = row.head(0);
-		// 1. critical part: the neighbours completed at the last step
-		T nu = lds(own + row.head(1));
-		T nl = lds(own + row.head(2));
-		if constexpr (SH == kAnyShape) {  // no such neighbour (its zero times inf is no zero)
-			nu = P1 > 1 ? nu : T(0);
-			nl = P2 > 1 ? nl : T(0);
-		}
-		Acc<T, KAHAN> a0 = acc[0];
-#pragma unroll
-		for (int r = 0; r + 1 < K0; ++r) acc[r] = acc[r + 1];
+		// 1. the point: the parts of its slice, group 1's sum
 		if constexpr (G > 1) {
 			const Hand& h = hand[((u & 1) ^ 1) * kThreads];
-			acc[K0 - 1].s = h[0];
-			if constexpr (KAHAN) acc[K0 - 1].c = h[1];
-		} else {
-			acc[K0 - 1].zero();
+			acc[K0 - 1].s = h[1];
+			if constexpr (KAHAN) acc[K0 - 1].c = h[2];
+			acc[K0 - 1].add(fma(c00[K0], zl, h[0]));
 		}
+		T part[K0];
+		parts_of(KC{}, coef, creg, part, ph, row);
+		acc[0].add(part[0]);
 		// slice t = s - lx - ly; slices before the first come out as zero (zero
 		// noise, sums and neighbours), and what lanes outside the grid or past
 		// the last slice compute reaches no lane that is in it
-		a0.add(fma(n010, nu, n001 * nl));
-		T z = eps + (a0.value() + n000 * eps);
+		T z = eps + (acc[0].value() + c00[0] * eps);
 		// slices t < t0 are given (a realtime stream's history): they feed the
 		// sums of later slices unchanged
 		if constexpr (!kSteady) z = s - lx - ly < t0 ? eps : z;
@@ -859,9 +851,14 @@ __device__ __forceinline__ void wave_tile(
 			*(active && unsigned(ts) < unsigned(nt) ? zeta + size_t(ts) * sxy + own_off : my_sink) = zd;
 			coherent_store(my_mbox + (my_m >= 0 ? size_t(u) * NB : 0), z);
 		}
-		// 4. everything else of the next point
-		if constexpr (P0 > 1) acc[0].add(n100 * z);
-		bulk_of(KC{}, coef, creg, acc, ph, row);
+		// 4. the point completes the sums of the slices after it
+#pragma unroll
+		for (int r = 1; r < K0; ++r) {
+			acc[r].add(fma(c00[r], z, part[r]));
+			acc[r - 1] = acc[r];
+		}
+		acc[K0 - 1].zero();
+		zl = z;
 		pin(acc);
 		if constexpr (!kConst) {
 			ph = pn;

@@ -34,7 +34,7 @@ const void* wave_kernel_of(const WaveVariant& v) {
 		if (v.buf && v.groups == 2) {
 			if constexpr (two_columns_fit(es, P0))
 				if (v.shape == kTwoColumns)
-					return fn(&ar_wave_kernel<T, 16, P0, KAHAN, 2, 2 * P0, kTwoColumns, true>);
+					return fn(&ar_wave_kernel<T, 16, P0, KAHAN, 2, 2 * P0 - 1, kTwoColumns, true>);
 			if (v.shape == kSquare)
 				return fn(&ar_wave_kernel<T, 16, P0, KAHAN, 2, square_taps(es, P0), kSquare, true>);
 			return fn(&ar_wave_kernel<T, 16, P0, KAHAN, 2, 0, kAnyShape, true>);

@@ -85,39 +85,32 @@ void append_tables(const double* phi, int P0, int P1, int P2, int P0S, int group
 	const int K0 = groups == 1 ? P0S : group_split(sizeof(T), P0S, shape);
 	const int P12 = P1 * P2;
 	const int chunk = chunk_taps(sizeof(T), group_most(sizeof(T), P0S, groups, shape));
-	const int ntap = padded_taps(P12, ntr, chunk);
-	auto at = [&](int k, int i, int j) {
-		return k < P0 && i < P1 && j < P2 ? T(phi[(size_t(k) * P1 + i) * P2 + j]) : T(0);
-	};
+	const int ntap = padded_taps(P12 - 1, ntr, chunk);
+	auto at = [&](int k, int m) { return k < P0 ? T(phi[size_t(k) * P12 + m]) : T(0); };
 	const size_t base = ph.size();
 	ph.resize(base + kNear + size_t(ntap) * P0S, T(0));
-	ph[base] = at(0, 0, 0);
-	ph[base + 1] = at(1, 0, 0);
-	ph[base + 2] = at(0, 1, 0);
-	ph[base + 3] = at(0, 0, 1);
-	auto lag = [](int i, int j) { return i + j >= 2 ? 0 : 2 - (i + j); };
-	for (int m = 0; m < P12; ++m) {
-		const int i = m / P2, j = m % P2;
-		for (int r = 0; r < P0S; ++r) {
-			const size_t e = r < K0 ? size_t(m) * K0 + r
-			                        : size_t(ntap) * K0 + size_t(m) * (P0S - K0) + (r - K0);
-			ph[base + kNear + e] = at(r + lag(i, j), i, j);
-		}
-	}
+	for (int k = 0; k < P0S; ++k) ph[base + k] = at(k, 0);
+	for (int e = 0; e < P12 - 1; ++e)
+		for (int k = 0; k < P0S; ++k)
+			ph[base + kNear + (k < K0 ? size_t(e) * K0 + k
+			                          : size_t(ntap) * K0 + size_t(e) * (P0S - K0) + (k - K0))] =
+				at(k, e + 1);
 	// keep every surface's block 16-element aligned
 	ph.resize((ph.size() + 15) / 16 * 16, T(0));
-	// a tap of distance d = max(i + j, 2) was completed d - 1 steps before this
+	// a tap of distance d = i + j was completed d steps before this; the padding
+	// repeats the last tap, so that its zero coefficients meet no value that the
+	// point does not depend on
 	const int R = ring_planes(P1, P2), es = int(sizeof(T));
 	const int WY = ring_pitch(es, TX, P1, P2, groups), plane = (TX + P1 - 1) * WY * es;
 	for (int s = 0; s < R; ++s) {
 		auto back = [&](int steps) { return ((s - steps) % R + R) % R * plane; };
 		offs.push_back(back(0));
-		offs.push_back(P1 > 1 ? back(1) - WY * es : back(0));
-		offs.push_back(P2 > 1 ? back(1) - es : back(0));
+		offs.push_back(back(1));
 		offs.push_back(0);
-		for (int m = 0; m < ntap; ++m) {
-			const int i = m < P12 ? m / P2 : 0, j = m < P12 ? m % P2 : 0;
-			offs.push_back(back(std::max(i + j, 2) - 1) - (i * WY + j) * es);
+		offs.push_back(0);
+		for (int e = 0; e < ntap; ++e) {
+			const int m = std::min(e + 1, P12 - 1), i = m / P2, j = m % P2;
+			offs.push_back(back(i + j) - (i * WY + j) * es);
 		}
 	}
 }
@@ -126,7 +119,7 @@ void append_tables(const double* phi, int P0, int P1, int P2, int P0S, int group
 constexpr size_t tile_lds(int es, int TX, int P1, int P2, int G, bool kahan) {
 	const int TY = kThreads / TX;
 	return size_t(es) * (size_t(ring_planes(P1, P2)) * (TX + P1 - 1) * ring_pitch(es, TX, P1, P2, G) +
-	                     size_t(TY + 1) * kThreads + (G > 1 ? 2 * kThreads * (kahan ? 2 : 1) : 0));
+	                     size_t(TY + 1) * kThreads + (G > 1 ? 2 * kThreads * (kahan ? 3 : 2) : 0));
 }
 
 // Every order whose halo a tile's width admits (ar_batch_fits) has its LDS, beside
@@ -196,10 +189,11 @@ void launch_kernel(const void* fn, int grid, int threads, size_t lds, hipStream_
 }
 
 // The form of a surface's tile.  Two groups of waves always paid where they
-// were measured (one lane per column: 1024 x 256 x 256 FP64 (7, 7, 2) 1.25 ms
-// against 0.83); resident coefficients where the shape of phi is one that the
-// fitted models have, P0 x P0 x 2 or P0 x P0 x P0 (streamed: (5, 5, 5) 1.5 times
-// as long).  Beyond a buffer descriptor's reach, and of order 1 in t, one group.
+// were measured (one lane per column: 1024 x 256 x 256 FP64 (7, 7, 2) 1.92 ms
+// against 0.84); resident coefficients where the shape of phi is one that the
+// fitted models have, P0 x P0 x 2 or P0 x P0 x P0 (streamed: that 1.34 ms, and FP32
+// (5, 5, 5) 1.7 times as long).  Beyond a buffer descriptor's reach, and of order 1
+// in t, one group.
 WaveVariant wave_variant(int es, int P0, int P1, int P2, bool buf) {
 	WaveVariant v;
 	v.buf = buf;
@@ -207,7 +201,7 @@ WaveVariant wave_variant(int es, int P0, int P1, int P2, bool buf) {
 	v.groups = 2;
 	if (P1 == P0 && P2 == 2 && two_columns_fit(es, P0)) {
 		v.shape = kTwoColumns;
-		v.ntr = 2 * P0;
+		v.ntr = 2 * P0 - 1;
 	} else if (P1 == P0 && P2 == P0) {
 		v.shape = kSquare;
 		v.ntr = square_taps(es, P0);
@@ -283,7 +277,7 @@ struct WavePlan {
 		var = wave_variant(int(es), P0, P1, P2, buffer_fits(es, kTX, nx, ny, nY, total_u, NB));
 		// (as append_tables lays them out)
 		const int chunk = chunk_taps(int(es), group_most(int(es), P0, var.groups, var.shape));
-		const size_t ntap = size_t(padded_taps(P1 * P2, var.ntr, chunk));
+		const size_t ntap = size_t(padded_taps(P1 * P2 - 1, var.ntr, chunk));
 		coef_bytes = ((kNear + ntap * P0 + 15) / 16 * 16 * es + 255) / 256 * 256;
 		table_bytes = coef_bytes + size_t(ring_planes(P1, P2)) * (kOffHead + ntap) * sizeof(int);
 		// a zero word for out-of-range loads (and the check word) and, without
