@@ -494,6 +494,9 @@ int arma_hip_batch_create(arma_hip_ctx* ctx, const arma_batch_desc* desc, arma_h
 		b->noise = arma_hip::noise_batch_create(ctx, b->precision, b->members);
 		b->ar = arma_hip::ar_batch_create(ctx, b->precision, b->members, b->cfg);
 		b->rescale = arma_hip::rescale_batch_create(ctx, b->precision, b->members);
+		// uploads are only in the order of this context's stream, and the batch may be
+		// generated on any
+		ARMA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
 		*out = b.release();
 	});
 }

@@ -157,8 +157,9 @@ inline void* work_buffer(arma_hip_ctx* ctx, Scratch& s, size_t n) {
 	return ctx->borrow_base + at;
 }
 
-// Copies a small, caller-owned host buffer to the device in stream order; the
-// buffer may be changed on return.
+// Copies a small, caller-owned host buffer to the device in the order of the
+// context's stream; the buffer may be changed on return.  What is kept for other
+// streams needs a wait before it is handed out.
 void upload(arma_hip_ctx* ctx, void* dst, const void* src, size_t bytes);
 
 // Records msg as the calling thread's last error (arma_hip_last_error).
@@ -246,9 +247,10 @@ struct BatchArConfig {
 struct NoiseBatch;
 struct ArBatch;
 struct RescaleBatch;
-// Construction uploads every table and allocates every buffer; the launches
-// only enqueue kernels on the context stream (no allocation, no host wait),
-// so they can be captured into a graph.
+// Construction allocates every buffer and uploads every table, in the order of the
+// context's stream (arma_hip_batch_create waits for them; a server's lane builds and
+// launches on one stream).  The launches only enqueue kernels on the context
+// stream (no allocation, no host wait), so they can be captured into a graph.
 NoiseBatch* noise_batch_create(arma_hip_ctx* ctx, int precision,
                                const std::vector<BatchMember>& m);
 void noise_batch_launch(arma_hip_ctx* ctx, NoiseBatch* b, void* arena);

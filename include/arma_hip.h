@@ -404,6 +404,8 @@ typedef struct arma_batch_trial {
 
 typedef struct arma_hip_batch arma_hip_batch;
 
+/* Waits for the context stream: the batch's tables are on the device when
+   this returns, and any context of that device may generate the batch. */
 int arma_hip_batch_create(arma_hip_ctx* ctx, const arma_batch_desc* desc, arma_hip_batch** out);
 void arma_hip_batch_destroy(arma_hip_batch* batch);
 /* offsets[n_surfaces + 1]: the first arena element of every surface, then
