@@ -43,7 +43,7 @@ __global__ __launch_bounds__(kThreads * G, G == 1 ? 1 : DENSE ? 4 : 2) void ar_b
 #define ARMA_BATCH_TILE(P, N, S)                                                              \
 	wave_tile<T, TX, P, KAHAN, G, N, S, BUF>(z, sf.nt, sf.nx, sf.ny, c0, c0 + kNear, tp, sf.P1, \
 	                                         sf.P2, sf.nY, zero, sink, mb, sf.NB,             \
-	                                         sf.total_steps, sf.t0, b, abortw, limit, nullptr, \
+	                                         sf.total_steps, sf.t0, b, BatchWait{abortw, limit},  \
 	                                         smem_raw)
 #define ARMA_BATCH_BODY(I)                                                                    \
 	case I:                                                                                   \

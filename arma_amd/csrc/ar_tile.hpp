@@ -374,19 +374,56 @@ __host__ __device__ inline int diagonal_tile(int b, int nX, int nY) {
 	return X * nY + Y;
 }
 
+// How long a tile waits for a neighbour's value; gives_up after poll n of a wait
+// that began with start = 0.
+//
+// The batch kernel's: every 256 polls it gives up once *abortw is set, or sets
+// *abortw itself when it has spun for more than limit ticks of the constant-rate
+// wall clock.  The host reads *abortw afterwards.
+struct BatchWait {
+	int* abortw;
+	long long limit;
+	__device__ __forceinline__ bool gives_up(int n, long long& start) {
+		if ((n & 255) != 0 || limit <= 0) return false;
+		if (__hip_atomic_load(abortw, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return true;
+		const long long now = wall_clock64();
+		if (start == 0) {
+			start = now;
+		} else if (now - start > limit) {
+			__hip_atomic_store(abortw, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+			return true;
+		}
+		return false;
+	}
+};
+
+// A single surface's: for ever, but in a checked launch limit polls, once per wave
+// and tile, since later waits of a wave that gave up end with their first.  Then
+// *check is set.  (Nothing more is in the loop, which is unrolled with the steps: with
+// the clock and *abortw in it a step took 2 % longer, at order 1 in t 10 %.)
+struct CheckedWait {
+	int* check;
+	int limit;  // 0: none
+	__device__ __forceinline__ bool gives_up(int n, long long&) {
+		if (n != limit) return false;
+		limit = 1;
+		__hip_atomic_store(check, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		return true;
+	}
+};
+
 // The march of one tile over all of t (P0 accumulators; a surface of lower
 // order in t has zero coefficients past its own order).  G groups of 256 lanes;
 // the first NTR taps resident.  With SH = kTwoColumns (all taps resident) LDS
 // offsets are constants of the step's phase, and the steady steps are unrolled
 // over the phases; with SH = kSquare the taps of one distance i + j share a
 // base that turns with the step, at constant offsets.
-template <class T, int TX, int P0, bool KAHAN, int G, int NTR, TapShape SH, bool BUF>
+template <class T, int TX, int P0, bool KAHAN, int G, int NTR, TapShape SH, bool BUF, class Wait>
 __device__ __forceinline__ void wave_tile(
 	T* __restrict__ zeta, int nt, int nx, int ny, const T* __restrict__ near,
 	const T* __restrict__ coef, const int* __restrict__ offs, int P1_, int P2_, int nY,
 	const T* __restrict__ zero, T* __restrict__ sink, T* __restrict__ mbox, int NB,
-	int total_steps, int t0, int b, int* abortw, long long limit, int* check,
-	unsigned char* smem_raw) {
+	int total_steps, int t0, int b, Wait wait, unsigned char* smem_raw) {
 	constexpr int kTX = TX, kTY = kThreads / TX;
 	static_assert(kTX * kTY == kThreads && kTX >= 8 && kTY >= 8, "tile shape");
 	static_assert(G == 1 || P0 > 1, "two groups need two accumulators");
@@ -711,10 +748,8 @@ __device__ __forceinline__ void wave_tile(
 	// A halo value that its producer has not stored yet reads as the sentinel
 	// that the launch filled the mailboxes with: the lane reads it again until
 	// it is there.  Rarely entered once a tile has fallen far enough behind its
-	// neighbours.  With limit > 0 the wait is bounded: every 256 polls it gives
-	// up once *abortw is set, or sets *abortw itself when it has spun for more
-	// than limit ticks of the constant-rate wall clock.  A launch that gave up
-	// still runs every tile to its end; the host reads *abortw afterwards.
+	// neighbours.  Where the wait is bounded it may end without the value; a launch
+	// that gave up still runs every tile to its end.
 	auto await_halo = [&](int u, T& h0, T& h1) {
 		long long start = 0;
 		for (int n = 1; __any(is_sentinel(h0) || is_sentinel(h1)); ++n) {
@@ -728,21 +763,9 @@ __device__ __forceinline__ void wave_tile(
 				if (w0) h0 = coherent_load(halo_at(0, u));
 				if (w1) h1 = coherent_load(halo_at(1, u));
 			}
-			if ((n & 255) == 0 && limit > 0) {
-				bool stop = __hip_atomic_load(abortw, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
-				const long long now = wall_clock64();
-				if (start == 0) {
-					start = now;
-				} else if (now - start > limit) {
-					__hip_atomic_store(abortw, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-					stop = true;
-				}
-				if (stop) break;
-			}
+			if (wait.gives_up(n, start)) break;
 			__builtin_amdgcn_s_sleep(1);
 		}
-		if (check && (is_sentinel(h0) || is_sentinel(h1)))
-			__hip_atomic_store(check, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 	};
 	// loads of step u2 (in order of u2); steady: every slice involved is in the
 	// grid, else each lane checks its own

@@ -15,14 +15,14 @@ __global__ __launch_bounds__(kThreads * G, G == 1 ? 1 : is_dense(sizeof(T), P0, 
 	T* __restrict__ zeta, int nt, int nx, int ny, const T* __restrict__ near,
 	const T* __restrict__ coef, const int* __restrict__ offs, int P1, int P2, int nY,
 	const T* __restrict__ zero, T* __restrict__ sink, T* __restrict__ mbox, int NB,
-	int total_steps, int* check) {
+	int total_steps, int* check, int limit) {
 	extern __shared__ __align__(16) unsigned char smem_raw[];
-	// unbounded waits: tiles wait only on tiles with smaller workgroup ids,
-	// which were dispatched before them
+	// tiles wait only on tiles with smaller workgroup ids, which were dispatched
+	// before them
 	wave_tile<T, TX, P0, KAHAN, G, NTR, SH, BUF>(zeta, nt, nx, ny, near, coef, offs, P1, P2, nY,
 	                                             zero, sink, mbox, NB, total_steps, 0,
 	                                             diagonal_tile(blockIdx.x, (nx + TX - 1) / TX, nY),
-	                                             nullptr, 0, check, smem_raw);
+	                                             CheckedWait{check, limit}, smem_raw);
 }
 
 // The single-surface kernel of order P0 in t for a variant.

@@ -155,15 +155,21 @@ void fill_mailboxes(hipStream_t stream, T* mbox, size_t n) {
 
 // Checked launches of single surfaces: ARMA_HIP_CHECK_HALO set (and not "0")
 // in the environment.  arm() points the kernel at a check word in the launch's
-// cleared zero-word line; verify() reads the word back after the launch and
-// fails the call if a consumer went on with a value that its producer had not
-// stored.
+// cleared zero-word line; verify() reads the word back after the launch and fails
+// the call if it was set.  The one-lane tile sets it when a halo value has not been
+// stored after kCheckPolls polls (ARMA_HIP_CHECK_HALO_POLLS: another number) instead of
+// waiting for it for ever; the quad tile, whose mailboxes are filled only in a
+// checked launch, when a consumer reads one that its producer has not stored.
+constexpr int kCheckPolls = 1 << 23;  // some ten seconds
 struct HaloCheck {
 	int* word = nullptr;
+	int limit = 0;
 	void arm(unsigned char* zero_line) {
 		const char* e = std::getenv("ARMA_HIP_CHECK_HALO");
 		if (!e || !*e || (e[0] == '0' && e[1] == 0)) return;
 		word = reinterpret_cast<int*>(zero_line + 128);
+		const char* polls = std::getenv("ARMA_HIP_CHECK_HALO_POLLS");
+		limit = polls && std::atoi(polls) > 0 ? std::atoi(polls) : kCheckPolls;
 	}
 	void verify(arma_hip_ctx* ctx) const {
 		if (!word) return;
@@ -171,7 +177,7 @@ struct HaloCheck {
 		ARMA_HIP_CHECK(hipMemcpyAsync(&v, word, sizeof v, hipMemcpyDeviceToHost, ctx->stream));
 		ARMA_HIP_CHECK(hipStreamSynchronize(ctx->stream));
 		ARMA_HIP_REQUIRE(v == 0, ARMA_HIP_ERUNTIME,
-		                 "checked launch: a halo value was read before its producer stored it");
+		                 "checked launch: a halo value was not there when it was needed");
 	}
 };
 
@@ -328,7 +334,7 @@ void launch_typed(arma_hip_ctx* ctx, const arma_ar_desc* d, T* zeta) {
 	launch_kernel(fn, p.ntiles, kThreads * p.var.groups, lds, ctx->stream, zeta, nt, nx, ny,
 	              (const T*)dbuf, (const T*)dbuf + kNear, (const int*)(dbuf + p.coef_bytes), P1, P2,
 	              p.nY, (const T*)fb, (T*)(fb + (p.var.buf ? 0 : 256)), mbox, p.NB, p.total_steps,
-	              hc.word);
+	              hc.word, hc.limit);
 	hc.verify(ctx);
 }
 
