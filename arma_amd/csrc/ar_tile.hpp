@@ -164,8 +164,9 @@ __device__ __forceinline__ void buffer_store(__amdgpu_buffer_rsrc_t r, unsigned 
 }
 
 // Every mailbox is filled with this signalling NaN before a launch; arithmetic
-// only produces quiet NaNs, so a consumer that reads it for a slice in range has
-// read a mailbox row before its producer stored it.
+// only produces quiet NaNs, and given values are stored there without it
+// (quieted), so a consumer that reads it for a slice in range has read a mailbox
+// row before its producer stored it.
 constexpr unsigned long long kHaloSentinel64 = 0x7ff4a5a5a5a5a5a5ull;
 constexpr unsigned kHaloSentinel32 = 0x7fa5a5a5u;
 
@@ -174,6 +175,13 @@ __device__ __forceinline__ bool is_sentinel(double v) {
 	return unsigned(__double2hiint(v)) == unsigned(kHaloSentinel64 >> 32);
 }
 __device__ __forceinline__ bool is_sentinel(float v) { return __float_as_uint(v) == kHaloSentinel32; }
+
+__device__ __forceinline__ double quieted(double v) {
+	return is_sentinel(v) ? __hiloint2double(__double2hiint(v) | 0x00080000, __double2loint(v)) : v;
+}
+__device__ __forceinline__ float quieted(float v) {
+	return is_sentinel(v) ? __uint_as_float(kHaloSentinel32 | 0x00400000u) : v;
+}
 
 // n elements at a 16-byte aligned address, 16 bytes per lane.
 template <class T>
@@ -846,8 +854,12 @@ __device__ __forceinline__ void wave_tile(
 		// the last slice compute reaches no lane that is in it
 		T z = eps + (acc[0].value() + c00[0] * eps);
 		// slices t < t0 are given (a realtime stream's history): they feed the
-		// sums of later slices unchanged
-		if constexpr (!kSteady) z = s - lx - ly < t0 ? eps : z;
+		// sums of later slices unchanged, but must not read as missing elsewhere
+		T zm = z;
+		if constexpr (!kSteady) {
+			z = s - lx - ly < t0 ? eps : z;
+			zm = t0 > 0 ? quieted(z) : z;
+		}
 		lds(own + here) = z;
 		// 2. halo values of step s
 		if (__any(is_sentinel(h0_q) || is_sentinel(h1_q))) await_halo(u, h0_q, h1_q);
@@ -868,11 +880,11 @@ __device__ __forceinline__ void wave_tile(
 			if constexpr (!kSteady) os = unsigned(ts) < unsigned(nt) ? os : kNone;
 			buffer_store<T>(surface(zstore), os, zd);
 			zstore += sxy;
-			buffer_store_coherent(mrsrc, moff, z);
+			buffer_store_coherent(mrsrc, moff, zm);
 			moff += mstep;
 		} else {
 			*(active && unsigned(ts) < unsigned(nt) ? zeta + size_t(ts) * sxy + own_off : my_sink) = zd;
-			coherent_store(my_mbox + (my_m >= 0 ? size_t(u) * NB : 0), z);
+			coherent_store(my_mbox + (my_m >= 0 ? size_t(u) * NB : 0), zm);
 		}
 		// 4. the point completes the sums of the slices after it
 #pragma unroll
