@@ -512,18 +512,19 @@ void build_part(arma_hip_ctx* ctx, const ArBatch* ab, ArBatchPart* pt,
 	upload(ctx, pt->queue.ptr, queue.data(), queue.size() * sizeof(int2));
 	// flags: the queue counter and the abort word (a line each), the quad tiles'
 	// progress counters, a zero word, and a sink for idle stores sized for the
-	// largest surface
+	// largest surface (behind buffer descriptors the one-lane tile stores none)
 	const size_t head = 256;
 	const size_t prog_bytes = pt->quad ? sizeof(int) * kProgStride * size_t(tiles) : 0;
 	const size_t zero_bytes = 256;
+	const size_t sink_lanes = pt->quad ? kQThreads : pt->buf ? 0 : kThreads;
 	unsigned char* fb = (unsigned char*)pt->flags.get(head + prog_bytes + zero_bytes +
-	                                                  size_t(max_tiles) * lanes * sizeof(T));
+	                                                  size_t(max_tiles) * sink_lanes * sizeof(T));
 	pt->clear_base = (int*)fb;
 	pt->next = (int*)fb;
 	pt->abortw = (int*)(fb + 128);
 	pt->progress = (int*)(fb + head);
 	pt->zero = fb + head + prog_bytes;
-	pt->sink = fb + head + prog_bytes + zero_bytes;
+	pt->sink = sink_lanes ? fb + head + prog_bytes + zero_bytes : pt->zero;
 	pt->nclear = (head + prog_bytes + zero_bytes) / sizeof(int);
 	pt->mbox_elems = size_t(mbox_elems);
 	pt->mbox.get(std::max<size_t>(size_t(mbox_elems), 64) * sizeof(T));
@@ -658,6 +659,7 @@ ArBatch* ar_batch_create(arma_hip_ctx* ctx, int precision, const std::vector<Bat
 
 ArBatch* ar_batch_new() { return new ArBatch; }
 
+// (a sink is counted for every member: whether there is one depends on the others)
 size_t ar_batch_member_bytes(const arma_ar_desc* d, int tile_x) {
 	const int TX = tile_x, TY = kThreads / TX;
 	const size_t es = d->precision == ARMA_FP32 ? 4 : 8;

@@ -43,3 +43,19 @@ def test_widest_orders(hip_ctx, tile_x, pshape, prec):
         # 10 columns of a row are wider than 8 + 1
         assert widths == ({8, 16} if pshape[2] == 10 else {8, 16, 32})
     batch.close()
+
+
+def test_device_bytes_of_many_tiles(hip_ctx):
+    """A batch holds its mailboxes and little else: no slots for stores that its
+    kernels do not make."""
+    shape, es = (1, 2048, 4096), 8
+    tiles = shape[1] // 16 * (shape[2] // 16)
+    # rows of 16 + 15 boundary values at 1 + 30 + 2 steps
+    mailboxes = tiles * (shape[0] + 32) * 31 * es
+    d = made(hip_ctx, shape, (2, 2, 2), arma_amd.FP64)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    batch = hip_ctx.batch([d], None, arma_amd.FP64)
+    used = before - torch.cuda.mem_get_info()[0]
+    batch.close()
+    assert mailboxes <= used <= mailboxes + (64 << 20)
