@@ -1440,8 +1440,6 @@ bool jump_fits(const arma_mt_params* mts, int n) {
 
 // Rows a segmented launch aims at (two workgroups of 16 rows per CU), the
 // most segments of one stream, and the shortest segment in words.
-// Rows a segmented launch aims at (two workgroups of 16 rows per CU), the
-// most segments of one stream, and the shortest segment in words.
 constexpr int kSegRowsPerCu = 32, kMaxSegments = 256, kMinSegmentWords = 1024;
 // Measured on MI355X, in ns: per word of a row filling its block and counting
 // (one workgroup of rows per CU), the jump's fixed part, each of its levels
@@ -1456,7 +1454,7 @@ SegmentPlan plan_segments(const arma_hip_ctx* ctx, int sem, int nstreams, long l
 	const int wpa = sem == ARMA_NOISE_DOUBLE ? 4 : 2;
 	const int rows = kSegRowsPerCu * std::max(ctx->num_cus, 1);
 	const int most = std::min(kMaxSegments, rows / std::max(nstreams, 1));
-	if (!small_blocks || most < 2 || !jump_fits(mts, nstreams)) return seg;
+	if (!small_blocks || most < 2) return seg;
 	// segment lengths e0 2^q, whole rounds of words: the shortest that keeps
 	// the launch within rows
 	for (int q = 2; q < 40; ++q)
@@ -1482,7 +1480,8 @@ SegmentPlan plan_segments(const arma_hip_ctx* ctx, int sem, int nstreams, long l
 			// one stream of 32768 normals: 146 us cut in 82 against 905 whole;
 			// 1000 of 73728: 0.79 against 2.12 ms; 2700 of 8192, which this
 			// line leaves whole, 279 against 241 us
-			if (k < 2 || cut > 0.93 * whole) return SegmentPlan();
+			// (the records last: there may be thousands)
+			if (k < 2 || cut > 0.93 * whole || !jump_fits(mts, nstreams)) return SegmentPlan();
 			return seg;
 		}
 	return SegmentPlan();
@@ -1491,18 +1490,25 @@ SegmentPlan plan_segments(const arma_hip_ctx* ctx, int sem, int nstreams, long l
 // Streams of large states take their words from noise_words_kernel when they
 // have at least kAheadNormals normals (below, the extra launches cost what the
 // stream does) and all words fit kAheadBytes, or in a batch, whose requests a
-// server admits by bytes that do not count them, kBatchAheadBytes.
+// server admits by bytes that do not count them, kBatchAheadBytes.  Beyond a stream per
+// CU its workgroups, which fill most of a CU's LDS and seed their state word by
+// word, run one after another, and the one-workgroup streams, four to a CU, are the
+// faster ones up to so many normals per state word (us, whole against ahead: MT19937,
+// 512 streams of 8192 132 and 118, 768 of 8192 140 and 153, 768 of 32768 403 and 333;
+// 1392 words of state, 256 of 8192 107 and 88, 512 of 8192 122 and 144, 512 of 32768
+// 285 and 264, 768 of 32768 321 and 380).
 constexpr long long kAheadNormals = 8192, kAheadBytes = 256ll << 20,
                     kBatchAheadBytes = 16ll << 20;
+constexpr int kAheadPerWord[] = {0, 16, 64, 64};  // by streams per CU, rounded up, less one
 
 WordPlan plan_ahead(const arma_hip_ctx* ctx, int sem, int nstreams, long long n,
                     const arma_mt_params* mts, bool small_blocks, long long most) {
 	WordPlan wp;
+	const int cus = std::max(ctx->num_cus, 1);
+	if (!small_blocks || n < kAheadNormals || nstreams > 4 * cus) return wp;
 	int nn_max = 0;
 	for (int i = 0; i < nstreams; ++i) nn_max = std::max(nn_max, int(mts[i].nn));
-	if (!small_blocks || nn_max <= 64 || n < kAheadNormals ||
-	    nstreams > 4 * std::max(ctx->num_cus, 1))
-		return wp;
+	if (nn_max <= 64 || n < (long long)kAheadPerWord[(nstreams - 1) / cus] * nn_max) return wp;
 	const int wpa = sem == ARMA_NOISE_DOUBLE ? 4 : 2;
 	// 4 / pi attempts per pair on average, in whole blocks
 	const long long blocks = (n * 41722 / 65536 + kBlockAttempts) / kBlockAttempts;
