@@ -50,6 +50,19 @@ struct Scratch {
 		}
 		return ptr;
 	}
+	// The same where the caller can do without: null when there is no memory.
+	void* try_get(size_t n) {
+		if (n > bytes) {
+			release();
+			if (hipMalloc(&ptr, n) != hipSuccess) {
+				(void)hipGetLastError();
+				ptr = nullptr;
+				return nullptr;
+			}
+			bytes = n;
+		}
+		return ptr;
+	}
 	void release() {
 		if (ptr) (void)hipFree(ptr);
 		ptr = nullptr;

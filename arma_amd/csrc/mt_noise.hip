@@ -1732,7 +1732,8 @@ void launch_white_noise(arma_hip_ctx* ctx, const arma_ar_desc* d, void* eps) {
 		                  (long long)std::min(g.part.x, g.shape.x) *
 		                      std::min(g.part.y, g.shape.y) * std::min(g.part.z, g.shape.z),
 		                  d->mts, small_blocks, kAheadBytes);
-	void* buf = plan.bytes(ntotal) ? ctx->noise_tmp.get(plan.bytes(ntotal)) : nullptr;
+	void* buf = plan.bytes(ntotal) ? ctx->noise_tmp.try_get(plan.bytes(ntotal)) : nullptr;
+	if (!buf) plan = NoisePlan();  // whole streams need no buffer
 	launch_by_type(ctx, fp32, sem, d->mts, dparams, dseeds, eps, g, ntotal, small_blocks, plan,
 	               buf);
 }
@@ -1850,7 +1851,8 @@ void noise_batch_build(arma_hip_ctx* ctx, NoiseBatch* b, int precision,
 			longest = std::max(longest, (long long)r.e0 * r.e1 * r.e2);
 		b->plan = plan_noise(ctx, b->sem, b->nstreams, longest, b->hparams.data(),
 		                     b->small_blocks, kBatchAheadBytes);
-		if (b->plan.bytes(b->nstreams)) b->parts.get(b->plan.bytes(b->nstreams));
+		if (b->plan.bytes(b->nstreams) && !b->parts.try_get(b->plan.bytes(b->nstreams)))
+			b->plan = NoisePlan();
 		b->params.get(sizeof(arma_mt_params) * recs.size());
 		b->seeds.get(sizeof(uint32_t) * recs.size());
 		b->recs.get(sizeof(NoiseBlockRec) * recs.size());

@@ -206,10 +206,11 @@ void launch_nit_realisation(arma_hip_ctx* ctx, void* zeta, size_t n, int precisi
 		}
 		if (levels < 4) levels = 0;
 	}
-	const int size = levels ? 1 << levels : 0;
+	int size = levels ? 1 << levels : 0;
 	double* table = nullptr;
+	if (size) table = (double*)ctx->nit_table.try_get(sizeof(double) * (size_t(size) + 1));
+	if (!table) size = 0;
 	if (size) {
-		table = (double*)ctx->nit_table.get(sizeof(double) * (size_t(size) + 1));
 		nit_table_kernel<<<size / 256 + 1, 256, 0, ctx->stream>>>(table, size, p);
 		ARMA_HIP_CHECK(hipGetLastError());
 	}
