@@ -23,7 +23,8 @@
 namespace arma_hip {
 namespace {
 
-constexpr size_t kNoAllocScratchBytes = size_t(32) << 20;
+// 32 MiB, and room for the coefficient and offset tables of the largest orders.
+constexpr size_t kNoAllocScratchBytes = (size_t(32) << 20) + (size_t(16) << 10);
 constexpr int kMaxDevices = 64;
 
 __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];

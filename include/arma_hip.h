@@ -153,7 +153,7 @@ int arma_hip_ar_generate(arma_hip_ctx* ctx, const arma_ar_desc* desc, void* zeta
    arma_hip_ar_generate with a device pointer zeta and algorithm
    ARMA_AR_WAVEFRONT, whose working buffers (MT records and seeds,
    coefficient tables, halo mailboxes) come from a
-   static device array of 32 MiB per GPU instead of allocations.  Returns
+   static device array of 32 MiB (and 16 KiB) per GPU instead of allocations.  Returns
    ARMA_HIP_EINVAL, before enqueuing anything, for a surface whose buffers
    exceed that (the mailboxes grow with tiles x (nt + 30 + order) x halo
    width).  All calls on one GPU share the array: calls that overlap on a GPU
