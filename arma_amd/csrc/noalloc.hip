@@ -3,19 +3,19 @@
 // arma_hip_ar_generate_noalloc is arma_hip_ar_generate (white noise, then
 // the wavefront recurrence, into a caller's device buffer) for callers that
 // cannot call hipMalloc: tight serving loops, harnesses that forbid
-// allocation.  (Its small host tables go up with a stream synchronisation, so
-// it is not meant for graph capture.)  Every buffer its kernels use beyond the
-// output (MT parameter records and seeds, coefficient and tap tables, tile
-// progress counters, the zero word, the store sink and the halo mailboxes)
-// is carved from `scratch`, a static device array of kNoAllocScratchBytes
+// allocation.  (Its host tables go up outside a graph, so it is not meant for
+// capture.)  Every buffer its kernels use beyond the
+// output (MT parameter records and seeds, coefficient and offset tables, the zero
+// word and the halo mailboxes; beyond a buffer descriptor's reach the store sink, on
+// the quad tile that and progress counters) is carved from `scratch`, a static device array of kNoAllocScratchBytes
 // that every GPU the library runs on holds until the process ends.  The
 // kernels are those of arma_hip_ar_generate, so the results are identical.
 //
 // Every call on a device shares that device's array: calls that overlap on
 // one GPU (several host threads, or several streams) race and must be
-// serialised by the caller.  What must start at zero (the progress counters
-// and the zero word) is cleared by a kernel on the caller's stream at every
-// call; everything else is written before it is read.
+// serialised by the caller.  What must start at a known value (the zero word, the
+// mailboxes' pattern, the quad tile's counters) is set by a kernel on the caller's
+// stream at every call; everything else is written before it is read.
 #include "common.hpp"
 
 #include <mutex>

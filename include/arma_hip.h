@@ -158,8 +158,8 @@ int arma_hip_ar_generate(arma_hip_ctx* ctx, const arma_ar_desc* desc, void* zeta
    exceed that (the mailboxes grow with tiles x (nt + 30 + order) x halo
    width).  All calls on one GPU share the array: calls that overlap on a GPU
    (other threads or streams) race, and the caller serialises them.  The
-   small host tables are uploaded with a stream synchronisation, so a call
-   cannot be captured into a HIP graph. */
+   host tables are uploaded outside any graph, so a call cannot be captured
+   into one. */
 int arma_hip_ar_generate_noalloc(arma_hip_ctx* ctx, const arma_ar_desc* desc, void* zeta);
 
 /* zeta *= sqrt(gamma0 / var(run)), where var is the sample variance of the
@@ -360,8 +360,10 @@ void arma_hip_partition_shape(const int32_t partition[3], const int32_t grid[3],
  * tile shape or the schedule.  A batch owns its device tables and scratch;
  * generate, capture and replay only enqueue kernels on the context stream.
  *
- * The recurrence launch is persistent: its workgroups wait on each other, so
- * all of them must be resident together.  Recurrence launches on one device
+ * The recurrence launch is persistent: its workgroups wait on each other.  The
+ * one-lane tile's take (surface, tile) entries in an order in which every entry
+ * only waits on earlier ones; the quad tile's (ARMA_HIP_QUAD_TILE) must all be
+ * resident together.  Recurrence launches on one device
  * therefore run one at a time, whatever context or stream enqueues them
  * (each waits for the previous one); noise, rescale and other work still
  * overlap.  A captured graph is outside that chain: do not replay it while
